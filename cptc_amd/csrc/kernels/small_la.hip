@@ -13,6 +13,7 @@
 
 #include "../host/hip_util.hpp"
 #include "../host/small_la.hpp"
+#include "block_sweep.hpp"
 
 namespace {
 
@@ -242,8 +243,7 @@ __global__ void hadamard_kernel(const double* A, const double* B, double* C, siz
 }
 
 // ---------------------------------------------------------------------------
-// pinv, fast path, one workgroup, A in LDS for R <= 128 (global scratch
-// otherwise):
+// pinv, fast path for R > 128, one workgroup, A in global scratch:
 //   1. blocked Cholesky A = L L^T: 16-column panels factored by wave 0
 //      (lanes over rows, no workgroup barrier inside a panel), then the
 //      trailing update by the whole workgroup;
@@ -298,12 +298,10 @@ __device__ inline double block_sum_all(double v, double* red)
 }
 
 __global__ __launch_bounds__(PINV_THREADS) void chol_inverse_kernel(const double* __restrict__ Ain,
-                                                                    int R, double* work,
+                                                                    int R, double* A,
                                                                     double* __restrict__ Ainv,
-                                                                    int* fallback, int use_lds)
+                                                                    int* fallback)
 {
-    extern __shared__ double lds[];
-    double* A = use_lds ? lds : work;
     __shared__ int ok;
     __shared__ double tau;
     __shared__ double xd[512];   // diagonal of X = L^-1 (R <= 512)
@@ -451,140 +449,200 @@ __global__ __launch_bounds__(PINV_THREADS) void chol_inverse_kernel(const double
 }
 
 // ---------------------------------------------------------------------------
-// pinv, fast path for R <= 64: one workgroup of SWEEP_T threads, the matrix
-// in registers.  Symmetric sweep (Beaton's SWEEP operator, i.e.
-// Gauss-Jordan elimination without pivoting in its symmetric form):
-// sweeping pivot k maps
-//   a_kk -> -1 / a_kk,  a_ik -> a_ik / a_kk  (i != k),
-//   a_ij -> a_ij - a_ik a_kj / a_kk          (i, j != k),
-// and after every pivot the matrix holds -A^-1.  The matrix stays
-// symmetric, so pivot row k is column k.  The pivots are the LDL^T pivots
-// (the squared Cholesky diagonal), so the fast-path test is the Cholesky
-// one: a pivot <= 1e-10 * max diag (or non-finite), or an inverse that
-// fails fast_inverse_ok, sets *fallback = 1 and leaves Ainv to the Jacobi
-// kernel.
-// Thread layout: RT >= R rows (16, 32 or 64), LPR = SWEEP_T / RT threads
-// per row, each holding C = RT / LPR consecutive columns: thread = row + RT
-// * part, columns part * C .. part * C + C - 1 (C = 1, 4, 16).  Per pivot
-// the threads owning column k write it to LDS (one slot per row) and every
-// thread reads its row's entry and its C columns' entries back.
+// pinv, fast path for R <= 128: the symmetric sweeps of block_sweep.hpp in
+// one workgroup, the matrix in registers.  A pivot <= 1e-10 * max diag (or
+// not finite), or an inverse that fails fast_inverse_ok, sets *fallback = 1.
+// Up to R = 64 the same workgroup then runs the Jacobi pseudoinverse
+// (jacobi_pinv_body, A in LDS, V in `V`: one launch per solve); above,
+// jacobi_pinv_kernel follows (the Jacobi path's registers would spill beside
+// the sweep's).  Bound by latency: R dependent scalar pivots.
 // ---------------------------------------------------------------------------
-constexpr int SWEEP_T = 256;
-
 template <int T>
 __device__ void jacobi_pinv_body(const double* __restrict__ Ain, int R, double* work, double* V,
                                  double* __restrict__ Ainv, int use_lds, double* lds);
 
-// When the fast path declines, the same workgroup runs the Jacobi
-// pseudoinverse (jacobi_pinv_body with its 256 threads, A in this kernel's
-// LDS, V in `V`), so R <= 64 needs one launch per solve, not two.
-template <int RT>
-__global__ __launch_bounds__(SWEEP_T) void sweep_inverse_kernel(const double* __restrict__ Ain,
-                                                                int R,
-                                                                double* __restrict__ Ainv,
-                                                                int* fallback, double* V)
+// A (R x R, R <= 16 M, row stride ld) swept in one wave, with no workgroup
+// barrier (the rest of the workgroup may do other work meanwhile).  Returns 1
+// with A^-1 stored to Ainv, or 0 when the fast path declines: the caller then
+// runs the Jacobi pseudoinverse.  Uniform over the wave.
+template <int M>
+__device__ int sweep_wave(const double* As, int ld, int R, double* __restrict__ Ainv)
 {
-    __shared__ double jA[RT * RT];   // the Jacobi path's A
-    constexpr int LPR = SWEEP_T / RT;
-    constexpr int C = RT / LPR;
-    static_assert(C >= 1 && C <= 16, "sweep layout");
-    __shared__ double col[RT];
-    __shared__ double wmax[SWEEP_T / WAVE];
-    __shared__ double wsum[SWEEP_T / WAVE];
-    const int tid = threadIdx.x;
-    const int row = tid % RT;
-    const int part = tid / RT;
-    const int c0 = part * C;
-    double a[C];
+    const int l = int(threadIdx.x) % WAVE, lr = l % 16, lk = l / 16;
+    cptc::bsweep::SweepWave<M> m;
 #pragma unroll
-    for (int c = 0; c < C; ++c)
-        a[c] = (row < R && c0 + c < R) ? Ain[size_t(row) * R + c0 + c] : 0.0;
-    // largest diagonal entry (the thread holding (row, row) contributes it)
-    // and ||A||_F^2
-    double md = 0.0, fa = 0.0;
+    for (int i = 0; i < M; ++i)
 #pragma unroll
-    for (int c = 0; c < C; ++c)
-    {
-        if (c0 + c == row) md = a[c];
-        fa += a[c] * a[c];
-    }
+        for (int j = 0; j < M; ++j)
+#pragma unroll
+            for (int v = 0; v < 4; ++v)
+                m.a[i][j][v] = As[min(16 * i + lk + 4 * v, R - 1) * ld + min(16 * j + lr, R - 1)];
+    double fa = 0.0, md = 0.0;
+#pragma unroll
+    for (int i = 0; i < M; ++i)
+#pragma unroll
+        for (int j = 0; j < M; ++j)
+#pragma unroll
+            for (int v = 0; v < 4; ++v)
+            {
+                const int r = 16 * i + lk + 4 * v, c = 16 * j + lr;
+                if (r >= R || c >= R) m.a[i][j][v] = 0.0;
+                fa += m.a[i][j][v] * m.a[i][j][v];
+                if (r == c) md = fmax(md, m.a[i][j][v]);
+            }
 #pragma unroll
     for (int o = WAVE / 2; o >= 1; o >>= 1)
     {
         md = fmax(md, __shfl_xor(md, o));
         fa += __shfl_xor(fa, o);
     }
-    if ((tid & (WAVE - 1)) == 0)
-    {
-        wmax[tid / WAVE] = md;
-        wsum[tid / WAVE] = fa;
-    }
-    __syncthreads();
-    double fro2_A = 0.0;
-#pragma unroll
-    for (int w = 0; w < SWEEP_T / WAVE; ++w)
-    {
-        md = fmax(md, wmax[w]);
-        fro2_A += wsum[w];
-    }
-    const double tau = 1e-10 * md;
-    int ok = (md > 0.0 && isfinite(md)) ? 1 : 0;
-#pragma unroll 1
-    for (int kp = 0; kp < LPR && kp * C < R && ok; ++kp)
-    {
-#pragma unroll
-        for (int kc = 0; kc < C; ++kc)
-        {
-            const int k = kp * C + kc;
-            if (k >= R || !ok) continue;   // uniform
-            if (part == kp) col[row] = a[kc];
-            __syncthreads();
-            const double p = col[k];
-            if (!(p > tau) || !isfinite(p))
-            {
-                ok = 0;   // every thread read the same pivot: uniform exit
-                continue;
-            }
-            const double ip = 1.0 / p;
-            const double f = col[row] * ip;    // a_ik / a_kk (1 on row k)
-            const bool prow = row == k;
-            const double g = prow ? 0.0 : f;
-            const double h = prow ? ip : 1.0;
-            double cj[C];
-#pragma unroll
-            for (int c = 0; c < C; ++c) cj[c] = col[c0 + c];
-#pragma unroll
-            for (int c = 0; c < C; ++c)
-            {
-                const double up = fma(-g, cj[c], a[c] * h);
-                a[c] = (c == kc && part == kp) ? (prow ? -ip : f) : up;
-            }
-            __syncthreads();
-        }
-    }
-    // both declines below are uniform over the workgroup
-    if (!ok)
-    {
-        if (tid == 0) *fallback = 1;
-        jacobi_pinv_body<SWEEP_T>(Ain, R, nullptr, V, Ainv, 1, jA);
-        return;
-    }
-    // condition check (fast_inverse_ok); padding entries are 0
+    if (!(md > 0.0) || !isfinite(md)) return 0;
+    int ok = 1;
+    m.template from<0>(R, lr, lk, 1e-10 * md, ok);
     double fi = 0.0;
 #pragma unroll
-    for (int c = 0; c < C; ++c) fi += a[c] * a[c];
-    const double fro2_inv = block_sum_all<SWEEP_T>(fi, wsum);
-    if (!fast_inverse_ok(fro2_A, fro2_inv, R))
+    for (int i = 0; i < M; ++i)
+#pragma unroll
+        for (int j = 0; j < M; ++j)
+#pragma unroll
+            for (int v = 0; v < 4; ++v) fi += m.a[i][j][v] * m.a[i][j][v];
+#pragma unroll
+    for (int o = WAVE / 2; o >= 1; o >>= 1) fi += __shfl_xor(fi, o);
+    if (!ok || !fast_inverse_ok(fa, fi, R)) return 0;
+#pragma unroll
+    for (int i = 0; i < M; ++i)
+#pragma unroll
+        for (int j = 0; j < M; ++j)
+#pragma unroll
+            for (int v = 0; v < 4; ++v)
+            {
+                const int r = 16 * i + lk + 4 * v, c = 16 * j + lr;
+                if (r < R && c < R) Ainv[size_t(r) * R + c] = -m.a[i][j][v];
+            }
+    return 1;
+}
+
+constexpr int SWEEP_T = 256;
+
+template <int M>
+__global__ __launch_bounds__(SWEEP_T) void sweep_wave_kernel(const double* __restrict__ Ain, int R,
+                                                             double* __restrict__ Ainv,
+                                                             int* fallback, double* V)
+{
+    __shared__ double jA[256 * M * M];   // the Jacobi path's A
+    __shared__ int okp;
+    if (threadIdx.x < WAVE)
+    {
+        const int ok = sweep_wave<M>(Ain, R, R, Ainv);
+        if (threadIdx.x == 0)
+        {
+            okp = ok;
+            *fallback = !ok;
+        }
+    }
+    __syncthreads();
+    if (!okp) jacobi_pinv_body<SWEEP_T>(Ain, R, nullptr, V, Ainv, 1, jA);
+}
+
+__global__ __launch_bounds__(SWEEP_T) void sweep_quad_kernel(const double* __restrict__ Ain, int R,
+                                                             double* __restrict__ Ainv,
+                                                             int* fallback, double* V)
+{
+    __shared__ double jA[64 * 64];   // the pivots' columns and rows, then the Jacobi path's A
+    __shared__ double red[SWEEP_T / WAVE], redm[SWEEP_T / WAVE];
+    static_assert(cptc::bsweep::QUAD_LDS <= 64 * 64, "pivot buffers");
+    const int tid = threadIdx.x, l = tid % WAVE, lr = l % 16, lk = l / 16;
+    const int w = __builtin_amdgcn_readfirstlane(tid / WAVE), wi = w / 2, wj = w % 2;
+    cptc::bsweep::SweepQuad m;
+    const int r0 = 32 * wi + lk, c0 = 32 * wj + lr;
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int j = 0; j < 2; ++j)
+#pragma unroll
+            for (int v = 0; v < 4; ++v)
+                m.a[i][j][v] = Ain[min(r0 + 16 * i + 4 * v, R - 1) * R + min(c0 + 16 * j, R - 1)];
+    double fa = 0.0, md = 0.0;
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int j = 0; j < 2; ++j)
+#pragma unroll
+            for (int v = 0; v < 4; ++v)
+            {
+                const int r = r0 + 16 * i + 4 * v, c = c0 + 16 * j;
+                const bool in = r < R && c < R;
+                if (!in) m.a[i][j][v] = r == c ? 1.0 : 0.0;
+                if (in) fa += m.a[i][j][v] * m.a[i][j][v];
+                if (in && r == c) md = fmax(md, m.a[i][j][v]);
+            }
+#pragma unroll
+    for (int o = WAVE / 2; o >= 1; o >>= 1) md = fmax(md, __shfl_xor(md, o));
+    if (l == 0) redm[w] = md;
+    const double fro2_A = block_sum_all<SWEEP_T>(fa, red);   // its barriers cover redm
+#pragma unroll
+    for (int q = 0; q < SWEEP_T / WAVE; ++q) md = fmax(md, redm[q]);
+    int ok = md > 0.0 && isfinite(md);
+    for (int h = 0; h < 2 && 32 * h < R; ++h)
+        m.from<0>(R, h, wi, wj, lr, lk, 1e-10 * md, jA, ok);   // every wave sees every pivot
+    double fi = 0.0;
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int j = 0; j < 2; ++j)
+#pragma unroll
+            for (int v = 0; v < 4; ++v)
+                if (r0 + 16 * i + 4 * v < R && c0 + 16 * j < R)
+                    fi += m.a[i][j][v] * m.a[i][j][v];
+    const double fro2_inv = block_sum_all<SWEEP_T>(fi, red);
+    if (!ok || !fast_inverse_ok(fro2_A, fro2_inv, R))   // uniform over the workgroup
     {
         if (tid == 0) *fallback = 1;
         jacobi_pinv_body<SWEEP_T>(Ain, R, nullptr, V, Ainv, 1, jA);
         return;
     }
     if (tid == 0) *fallback = 0;
-    if (row < R)
 #pragma unroll
-        for (int c = 0; c < C; ++c)
-            if (c0 + c < R) Ainv[size_t(row) * R + c0 + c] = -a[c];
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int j = 0; j < 2; ++j)
+#pragma unroll
+            for (int v = 0; v < 4; ++v)
+            {
+                const int r = r0 + 16 * i + 4 * v, c = c0 + 16 * j;
+                if (r < R && c < R) Ainv[size_t(r) * R + c] = -m.a[i][j][v];
+            }
+}
+
+template <int NB, int T>
+__global__ __launch_bounds__(T) void block_sweep_kernel(const double* __restrict__ Ain, int R,
+                                                        double* __restrict__ Ainv, int* fallback)
+{
+    extern __shared__ double lds[];
+    __shared__ double red[T / WAVE], redm[T / WAVE];
+    __shared__ int bad;
+    constexpr int W = T / WAVE;
+    const int tid = threadIdx.x, nb = (R + 15) / 16;
+    cptc::bsweep::Blocks<NB, W> m;
+    m.place(tid / WAVE, nb);
+    m.load(R, [&](int r, int c) { return Ain[size_t(r) * R + c]; });
+    double fa, md;
+    m.norms(R, fa, md);
+#pragma unroll
+    for (int o = WAVE / 2; o >= 1; o >>= 1) md = fmax(md, __shfl_xor(md, o));
+    if (tid % WAVE == 0) redm[tid / WAVE] = md;
+    if (tid == 0) bad = 0;
+    const double fro2_A = block_sum_all<T>(fa, red);   // its barriers cover redm and bad
+#pragma unroll
+    for (int w = 0; w < W; ++w) md = fmax(md, redm[w]);
+    const int okw = m.sweep(R, nb, 1e-10 * md, lds);
+    double fi, unused;
+    m.norms(R, fi, unused);
+    if (!okw && tid % WAVE == 0) bad = 1;
+    const double fro2_inv = block_sum_all<T>(fi, red);
+    const bool ok = !bad && md > 0.0 && isfinite(md) && fast_inverse_ok(fro2_A, fro2_inv, R);
+    if (tid == 0) *fallback = !ok;
+    if (ok) m.store(R, [&](int r, int c, double x) { Ainv[size_t(r) * R + c] = -x; });
 }
 
 // ---------------------------------------------------------------------------
@@ -1307,88 +1365,6 @@ __device__ __forceinline__ double upd3_keep(double v)
     return v;
 }
 
-// The pinv fast path of sweep_inverse_kernel run by one wave, with no
-// workgroup barrier (the rest of the workgroup does other work meanwhile):
-// A (R x R, row stride ld) read from LDS, lane l keeps row l % RT, columns
-// C (l / RT) .. + C - 1 (C = RT^2 / 64), the pivot column goes through the
-// LDS row colb (a wave's LDS accesses run in order).  Per entry the same
-// operations as sweep_inverse_kernel, so an accepted inverse is the same
-// bits.  Returns 1 with -(swept A) = A^-1 stored to Ainv, or 0 when a pivot
-// is <= 1e-10 max diag (or not finite) or fast_inverse_ok fails: the
-// caller then runs the Jacobi pseudoinverse.  Uniform over the wave.
-template <int RT>
-__device__ int sweep_wave(const double* As, int ld, int R, double* __restrict__ Ainv,
-                          double* colb)
-{
-    constexpr int LPR = WAVE / RT;
-    constexpr int C = RT / LPR;
-    const int l = int(threadIdx.x) % WAVE;
-    const int row = l % RT, part = l / RT, c0 = part * C;
-    double a[C];
-#pragma unroll
-    for (int c = 0; c < C; ++c) a[c] = (row < R && c0 + c < R) ? As[row * ld + c0 + c] : 0.0;
-    double md = 0.0, fa = 0.0;
-#pragma unroll
-    for (int c = 0; c < C; ++c)
-    {
-        if (c0 + c == row) md = a[c];
-        fa += a[c] * a[c];
-    }
-#pragma unroll
-    for (int o = WAVE / 2; o >= 1; o >>= 1)
-    {
-        md = fmax(md, __shfl_xor(md, o));
-        fa += __shfl_xor(fa, o);
-    }
-    const double tau = 1e-10 * md;
-    int ok = (md > 0.0 && isfinite(md)) ? 1 : 0;
-#pragma unroll 1
-    for (int kp = 0; kp < LPR && kp * C < R && ok; ++kp)
-    {
-#pragma unroll
-        for (int kc = 0; kc < C; ++kc)
-        {
-            const int k = kp * C + kc;
-            if (k >= R || !ok) continue;   // uniform
-            if (part == kp) colb[row] = a[kc];
-            __builtin_amdgcn_wave_barrier();
-            const double p = colb[k];
-            if (!(p > tau) || !isfinite(p))
-            {
-                ok = 0;
-                continue;
-            }
-            const double ip = 1.0 / p;
-            const double f = colb[row] * ip;
-            const bool prow = row == k;
-            const double g = prow ? 0.0 : f;
-            const double h = prow ? ip : 1.0;
-            double cj[C];
-#pragma unroll
-            for (int c = 0; c < C; ++c) cj[c] = colb[c0 + c];
-            __builtin_amdgcn_wave_barrier();
-#pragma unroll
-            for (int c = 0; c < C; ++c)
-            {
-                const double up = fma(-g, cj[c], a[c] * h);
-                a[c] = (c == kc && part == kp) ? (prow ? -ip : f) : up;
-            }
-        }
-    }
-    if (!ok) return 0;
-    double fi = 0.0;
-#pragma unroll
-    for (int c = 0; c < C; ++c) fi += a[c] * a[c];
-#pragma unroll
-    for (int o = WAVE / 2; o >= 1; o >>= 1) fi += __shfl_xor(fi, o);
-    if (!fast_inverse_ok(fa, fi, R)) return 0;
-    if (row < R)
-#pragma unroll
-        for (int c = 0; c < C; ++c)
-            if (c0 + c < R) Ainv[size_t(row) * R + c0 + c] = -a[c];
-    return 1;
-}
-
 constexpr int UPD3_T = 256;
 constexpr int UPD3_WAVES = UPD3_T / WAVE;
 constexpr int UPD3_MAX_ROWS = 4096;
@@ -1407,7 +1383,7 @@ __global__ __launch_bounds__(UPD3_T) void update3_small_kernel(
     constexpr int KS = 4 * NT;              // K steps of 4 over R padded to 16 NT
     __shared__ double gl[UPD3_WAVES][NP][256];
     __shared__ double g_s[32][33], f_s[32][33];
-    __shared__ double n_s[32], lamn_s[32], fit_s[UPD3_WAVES][32], fs_s[32], colb[32];
+    __shared__ double n_s[32], lamn_s[32], fit_s[UPD3_WAVES][32], fs_s[32];
     __shared__ double red2[UPD3_WAVES];
     __shared__ int last_s, decl_s;
     const int tid = threadIdx.x, w = tid / WAVE, l = tid % WAVE;
@@ -1654,7 +1630,7 @@ __global__ __launch_bounds__(UPD3_T) void update3_small_kernel(
     if (st < 0)
     {
         // wave 0: the next mode's pinv (one-wave sweep)
-        const int okp = sweep_wave<16 * NT>(&f_s[0][0], 33, R, Anext, colb);
+        const int okp = sweep_wave<NT>(&f_s[0][0], 33, R, Anext);
         if (l == 0) decl_s = !okp;
     }
     else
@@ -1730,7 +1706,7 @@ __global__ __launch_bounds__(UPD1_T) void update3_one_kernel(
     constexpr int KS = 4 * NT;
     __shared__ double gl[UPD1_WAVES][NP][256];
     __shared__ double g_s[32][33], f_s[32][33];
-    __shared__ double n_s[32], lamn_s[32], fit_s[UPD1_WAVES][32], colb[32];
+    __shared__ double n_s[32], lamn_s[32], fit_s[UPD1_WAVES][32];
     __shared__ double red2[UPD1_WAVES];
     __shared__ int decl_s;
     const int tid = threadIdx.x, w = tid / WAVE, l = tid % WAVE;
@@ -1928,7 +1904,7 @@ __global__ __launch_bounds__(UPD1_T) void update3_one_kernel(
     {
         if (Anext)
         {
-            const int okp = sweep_wave<16 * NT>(&f_s[0][0], 33, R, Anext, colb);
+            const int okp = sweep_wave<NT>(&f_s[0][0], 33, R, Anext);
             if (l == 0) decl_s = !okp;
         }
     }
@@ -2196,31 +2172,28 @@ namespace {
 int pinv_launch_ws(const double* d_FtF, double* d_Ainv, int R, int* flag, double* work,
                    double* V, hipStream_t s)
 {
-    const size_t RR = size_t(R) * R;
-    const bool use_lds = RR * sizeof(double) <= 128 * 1024;
-    const size_t lds = use_lds ? RR * sizeof(double) : 0;
-    static cptc::DeviceOnce attr;
-    CPTC_HIP(attr.lds_limit({reinterpret_cast<const void*>(chol_inverse_kernel),
-                             reinterpret_cast<const void*>(jacobi_pinv_kernel)},
-                            128 * 1024));
-    // R <= 64: the sweep kernel runs its own Jacobi fallback (one launch)
-    if (R <= 16)
-        hipLaunchKernelGGL(sweep_inverse_kernel<16>, dim3(1), dim3(SWEEP_T), 0, s, d_FtF, R, d_Ainv,
-                           flag, V);
-    else if (R <= 32)
-        hipLaunchKernelGGL(sweep_inverse_kernel<32>, dim3(1), dim3(SWEEP_T), 0, s, d_FtF, R, d_Ainv,
-                           flag, V);
-    else if (R <= 64)
-        hipLaunchKernelGGL(sweep_inverse_kernel<64>, dim3(1), dim3(SWEEP_T), 0, s, d_FtF, R, d_Ainv,
-                           flag, V);
-    else
+    if (R <= 64)
     {
-        hipLaunchKernelGGL(chol_inverse_kernel, dim3(1), dim3(PINV_THREADS), lds, s, d_FtF, R,
-                           work, d_Ainv, flag, int(use_lds));
+        auto kern = R <= 16   ? sweep_wave_kernel<1>
+                    : R <= 32 ? sweep_wave_kernel<2>
+                              : sweep_quad_kernel;
+        hipLaunchKernelGGL(kern, dim3(1), dim3(SWEEP_T), 0, s, d_FtF, R, d_Ainv, flag, V);
         CPTC_LAUNCHED();
-        hipLaunchKernelGGL(jacobi_pinv_kernel, dim3(1), dim3(PINV_THREADS), lds, s, d_FtF, R, work,
-                           V, d_Ainv, flag, int(use_lds));
+        return CPTC_OK;
     }
+    const bool use_lds = R <= 128;
+    static cptc::DeviceOnce attr;
+    CPTC_HIP(attr.lds_limit({reinterpret_cast<const void*>(jacobi_pinv_kernel)}, 128 * 1024));
+    if (use_lds)
+        hipLaunchKernelGGL((block_sweep_kernel<8, 768>), dim3(1), dim3(768),
+                           8 * cptc::bsweep::lds_doubles(8), s, d_FtF, R, d_Ainv, flag);
+    else
+        hipLaunchKernelGGL(chol_inverse_kernel, dim3(1), dim3(PINV_THREADS), 0, s, d_FtF, R, work,
+                           d_Ainv, flag);
+    CPTC_LAUNCHED();
+    hipLaunchKernelGGL(jacobi_pinv_kernel, dim3(1), dim3(PINV_THREADS),
+                       use_lds ? size_t(R) * R * sizeof(double) : 0, s, d_FtF, R, work, V, d_Ainv,
+                       flag, int(use_lds));
     CPTC_LAUNCHED();
     return CPTC_OK;
 }

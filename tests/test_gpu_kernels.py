@@ -549,6 +549,36 @@ def test_solve_pinv_spd(ca, dev, R):
     assert rel_err(out.numpy(), (Y @ inv) / lam) < 1e-9
 
 
+@pytest.mark.parametrize("R", [2, 15, 31, 34, 47, 48, 49, 79, 81, 96, 97, 112, 113, 127])
+def test_pinv_block_edges(ca, dev, R):
+    """The sweeps on both sides of their 16-row blocks and at odd R: the inverse
+    within the forward error of a backward-stable inverse (8 R kappa eps),
+    above R = 64 its off-diagonal blocks exact mirrors, and a matrix whose
+    only bad pivot is the last one (a copy of column 0) declined."""
+    rng = np.random.default_rng(7 * R)
+    Fa, Fb = rng.random((3 * R + 20, R)), rng.random((2 * R + 30, R))
+    A = (Fa.T @ Fa) * (Fb.T @ Fb)
+    path = zeros(ca, (1,), np.int32)
+    Ainv = zeros(ca, (R, R))
+    dA = to_dev(ca, A)
+    assert ca.lib.cptc_pinv_sym(dA.data_ptr(), Ainv.data_ptr(), R, path.data_ptr(),
+                                stream(ca)) == 0
+    ca.sync()
+    assert int(path.numpy()[0]) == 0
+    got = Ainv.numpy()
+    eps = np.finfo(np.float64).eps
+    assert rel_err(got, np.linalg.inv(A)) < 8 * R * np.linalg.cond(A) * eps
+    blk = np.arange(R) // 16
+    off = blk[:, None] != blk[None, :]
+    assert R <= 64 or np.array_equal(got[off], got.T[off])
+    Fa[:, R - 1], Fb[:, R - 1] = Fa[:, 0], Fb[:, 0]
+    dB = to_dev(ca, (Fa.T @ Fa) * (Fb.T @ Fb))
+    assert ca.lib.cptc_pinv_sym(dB.data_ptr(), Ainv.data_ptr(), R, path.data_ptr(),
+                                stream(ca)) == 0
+    ca.sync()
+    assert int(path.numpy()[0]) == 1
+
+
 @pytest.mark.parametrize("R", [24, 64, 100])
 def test_pinv_singular_takes_jacobi_path(ca, orc, dev, R):
     """Rank-deficient FtF: the fast path (register sweep for R <= 64, blocked

@@ -26,10 +26,13 @@
 #include <limits>
 #include <random>
 #include <string>
+#include <system_error>
+#include <thread>
 #include <vector>
 
 #include "blk3_params.hpp"
 #include "cptc_hip.h"
+#include "dev_pool.hpp"
 #include "hip_util.hpp"
 #include "host_util.hpp"
 #include "layout.hpp"
@@ -379,21 +382,22 @@ void destroy(Als3* h)
     if (!h) return;
     for (hipStream_t st : {h->s, h->s_pinv, h->s_dense})
         if (st) (void)hipStreamSynchronize(st);
+    PoolScope scope(nullptr, true);   // nothing is queued on the blocks any more
     free_partition(h->part);
     free_views(h->views);
     free_views(h->dviews);
     free_views(h->aviews);
     free_blk(h->blk);
     for (auto& p : h->d_perm)
-        if (p) (void)hipFree(p);
+        dev_free(p);
     for (int m = 0; m < 3; ++m)
         for (void* p : {(void*)h->d_order[m], (void*)h->d_goff[m]})
-            if (p) (void)hipFree(p);
+            dev_free(p);
     for (SplitImg& g : h->timg) free_split_img(g);
     for (void* p : {(void*)h->d_tile_f32, (void*)h->d_tile_ws, (void*)h->d_F, (void*)h->d_lambda, (void*)h->d_G,
                     (void*)h->d_FtF, (void*)h->d_Ainv, (void*)h->d_FtV, (void*)h->d_norms,
                     (void*)h->d_scal, (void*)h->d_fit_hist})
-        if (p) (void)hipFree(p);
+        dev_free(p);
     for (auto& e : h->ev)
         if (e) (void)hipEventDestroy(e);
     for (auto& e : h->kev)
@@ -428,8 +432,8 @@ int build_groups(Als3& h)
         const int cap = cptc::tile_group_cap(nt, h.R, h.num_cus, TILE_GROUP, h.tile_b3 ? 32 : 16);
         CPTC_TRY(cptc_dense_groups(h.part.h_tiles4.data(), 4, nt, m, cap, order.data(),
                                    goff.data(), &ng));
-        CPTC_HIP(hipMalloc(&h.d_order[m], nt * sizeof(uint32_t)));
-        CPTC_HIP(hipMalloc(&h.d_goff[m], (ng + 1) * sizeof(uint32_t)));
+        CPTC_TRY(dev_alloc(&h.d_order[m], nt * sizeof(uint32_t)));
+        CPTC_TRY(dev_alloc(&h.d_goff[m], (ng + 1) * sizeof(uint32_t)));
         CPTC_HIP(hipMemcpyAsync(h.d_order[m], order.data(), nt * sizeof(uint32_t),
                                 hipMemcpyHostToDevice, h.s));
         CPTC_HIP(hipMemcpyAsync(h.d_goff[m], goff.data(), (ng + 1) * sizeof(uint32_t),
@@ -439,6 +443,39 @@ int build_groups(Als3& h)
     }
     return CPTC_OK;
 }
+
+// The initial factors' values: one mt19937 sequence, U[0, 1) (~8 ns a draw:
+// 1.8 ms at 9 200 rows x 25, 50 ms at 50 000 x 128), drawn beside the rest of
+// the set-up, whose host side mostly waits for the device.
+struct FactorInit
+{
+    std::vector<double> values;
+    std::thread th;
+
+    static void fill(std::vector<double>& v, unsigned seed)
+    {
+        std::mt19937 gen(seed);
+        std::uniform_real_distribution<double> dis(0.0, 1.0);
+        for (double& x : v) x = dis(gen);
+    }
+    void start(size_t n, uint64_t seed)
+    {
+        values.resize(n);
+        try
+        {
+            th = std::thread([this, seed] { fill(values, unsigned(seed)); });
+        }
+        catch (const std::system_error&)   // no thread to be had
+        {
+            fill(values, unsigned(seed));
+        }
+    }
+    void finish()
+    {
+        if (th.joinable()) th.join();
+    }
+    ~FactorInit() { finish(); }
+};
 
 int create(const cptc_coo* coo, const cptc_als3_opts* opts, Als3* h)
 {
@@ -470,6 +507,9 @@ int create(const cptc_coo* coo, const cptc_als3_opts* opts, Als3* h)
                      (unsigned long long)mx, (unsigned long long)h->dims[m]);
     }
     CPTC_TRY(init_streams(*h));
+    PoolScope scope(h->s);   // the set-up's blocks: everything below runs on h->s
+    FactorInit init;
+    init.start((h->dims[0] + h->dims[1] + h->dims[2]) * size_t(o.R), o.seed);
     int dev = 0;
     CPTC_HIP(hipGetDevice(&dev));
     hipDeviceProp_t prop{};
@@ -493,26 +533,20 @@ int create(const cptc_coo* coo, const cptc_als3_opts* opts, Als3* h)
         {
             h->perm[m].resize(h->dims[m]);
             for (uint64_t x = 0; x < h->dims[m]; ++x) h->perm[m][x] = int32_t(x);
-            CPTC_HIP(hipMalloc(&h->d_perm[m], h->dims[m] * sizeof(int32_t)));
+            CPTC_TRY(dev_alloc(&h->d_perm[m], h->dims[m] * sizeof(int32_t)));
             CPTC_HIP(hipMemcpyAsync(h->d_perm[m], h->perm[m].data(), h->dims[m] * sizeof(int32_t),
                                     hipMemcpyHostToDevice, h->s));
         }
     }
 
-    // 2. factors in the relabelled space (common.cu:66-123, main.cu:228-264)
+    // 2. factors in the relabelled space (common.cu:66-123, main.cu:228-264):
+    // buffers now, values once init's thread has them (step 6)
     const int R = h->R;
     const size_t tot = (h->dims[0] + h->dims[1] + h->dims[2]) * size_t(R);
-    {
-        std::vector<double> hf(tot);
-        std::mt19937 gen(unsigned(o.seed));
-        std::uniform_real_distribution<double> dis(0.0, 1.0);
-        for (size_t x = 0; x < tot; ++x) hf[x] = dis(gen);
-        CPTC_HIP(hipMalloc(&h->d_F, tot * sizeof(double)));
-        CPTC_HIP(hipMemcpy(h->d_F, hf.data(), tot * sizeof(double), hipMemcpyHostToDevice));
-        h->F[0] = h->d_F;
-        h->F[1] = h->F[0] + h->dims[0] * R;
-        h->F[2] = h->F[1] + h->dims[1] * R;
-    }
+    CPTC_TRY(dev_alloc(&h->d_F, tot * sizeof(double)));
+    h->F[0] = h->d_F;
+    h->F[1] = h->F[0] + h->dims[0] * R;
+    h->F[2] = h->F[1] + h->dims[1] * R;
 
     // 3. hybrid partition, then the COO is released (main.cu:268-301)
     CPTC_TRY(partition3_device(c, o.threshold, h->num_cus, h->part, h->s));
@@ -526,12 +560,12 @@ int create(const cptc_coo* coo, const cptc_als3_opts* opts, Als3* h)
     for (int m = 0; m < 3; ++m)
         if (h->part.d_sp[m])
         {
-            CPTC_HIP(hipFree(h->part.d_sp[m]));
+            dev_free(h->part.d_sp[m]);
             h->part.d_sp[m] = nullptr;
         }
     if (h->part.d_sp_val)
     {
-        CPTC_HIP(hipFree(h->part.d_sp_val));
+        dev_free(h->part.d_sp_val);
         h->part.d_sp_val = nullptr;
     }
 
@@ -565,7 +599,7 @@ int create(const cptc_coo* coo, const cptc_als3_opts* opts, Als3* h)
     {
         if (h->use_mfma)
         {
-            CPTC_HIP(hipMalloc(&h->d_tile_f32, size_t(h->part.ntiles) * 4096 * sizeof(float)));
+            CPTC_TRY(dev_alloc(&h->d_tile_f32, size_t(h->part.ntiles) * 4096 * sizeof(float)));
             CPTC_TRY(cptc_dense_tiles_pack3(h->part.d_pool_lid, h->part.d_pool_val,
                                             h->part.d_pool_off, size_t(h->part.ntiles),
                                             h->d_tile_f32, h->s));
@@ -583,6 +617,11 @@ int create(const cptc_coo* coo, const cptc_als3_opts* opts, Als3* h)
     choose_tiles(*h);
     CPTC_TRY(build_groups(*h));
     CPTC_TRY(build_blk(*h));
+    // 6. the factors' values, before alloc_buffers reads them for ||X||^2; it
+    // waits for the stream, so init's vector outlives the copy
+    init.finish();
+    CPTC_HIP(hipMemcpyAsync(h->d_F, init.values.data(), tot * sizeof(double),
+                            hipMemcpyHostToDevice, h->s));
     CPTC_TRY(alloc_buffers(*h));
     choose_graph(*h);
     choose_small_update(*h);
@@ -608,7 +647,7 @@ int alloc_buffers(Als3& hr)
     if (h->tile_b3)
     {
         h->tile_ws_bytes = cptc_tile_operands_bytes(maxdim, R);
-        CPTC_HIP(hipMalloc(&h->d_tile_ws, h->tile_ws_bytes));
+        CPTC_TRY(dev_alloc(&h->d_tile_ws, h->tile_ws_bytes));
         // compacted split images, one per target mode: the kernel's A operand
         // halves of every 8-cell segment with a nonzero bit, read instead of
         // splitting the dense image on every launch
@@ -617,13 +656,13 @@ int alloc_buffers(Als3& hr)
             for (int m = 0; m < 3; ++m)
                 CPTC_TRY(build_split_img(h->d_tile_f32, size_t(h->part.ntiles), m, h->timg[m], h->s));
     }
-    CPTC_HIP(hipMalloc(&h->d_lambda, size_t(R) * sizeof(double)));
-    CPTC_HIP(hipMalloc(&h->d_G, 3 * RR * sizeof(double)));
-    CPTC_HIP(hipMalloc(&h->d_FtF, RR * sizeof(double)));
-    CPTC_HIP(hipMalloc(&h->d_Ainv, RR * sizeof(double)));
-    CPTC_HIP(hipMalloc(&h->d_FtV, maxdim * size_t(R) * sizeof(double)));
-    CPTC_HIP(hipMalloc(&h->d_norms, size_t(R) * sizeof(double)));
-    CPTC_HIP(hipMalloc(&h->d_scal, 4 * sizeof(double)));
+    CPTC_TRY(dev_alloc(&h->d_lambda, size_t(R) * sizeof(double)));
+    CPTC_TRY(dev_alloc(&h->d_G, 3 * RR * sizeof(double)));
+    CPTC_TRY(dev_alloc(&h->d_FtF, RR * sizeof(double)));
+    CPTC_TRY(dev_alloc(&h->d_Ainv, RR * sizeof(double)));
+    CPTC_TRY(dev_alloc(&h->d_FtV, maxdim * size_t(R) * sizeof(double)));
+    CPTC_TRY(dev_alloc(&h->d_norms, size_t(R) * sizeof(double)));
+    CPTC_TRY(dev_alloc(&h->d_scal, 4 * sizeof(double)));
     {
         std::vector<double> ones(size_t(R), 1.0);
         CPTC_HIP(hipMemcpyAsync(h->d_lambda, ones.data(), size_t(R) * sizeof(double),
@@ -1263,8 +1302,9 @@ extern "C" int cptc_als3_factor(void* handle, int mode, int unpermuted, double* 
         CPTC_HIP(hipStreamSynchronize(h->s));
         return CPTC_OK;
     }
+    cptc::PoolScope scope(h->s);
     double* tmp = nullptr;
-    CPTC_HIP(hipMalloc(&tmp, n * sizeof(double)));
+    CPTC_TRY(cptc::dev_alloc(&tmp, n * sizeof(double)));
     int rc = cptc_unpermute_factor(h->F[mode], tmp, h->d_perm[mode], h->dims[mode], h->R, h->s);
     if (rc == CPTC_OK)
     {
@@ -1273,7 +1313,7 @@ extern "C" int cptc_als3_factor(void* handle, int mode, int unpermuted, double* 
             hipStreamSynchronize(h->s) != hipSuccess)
             rc = CPTC_ERR_HIP;
     }
-    (void)hipFree(tmp);
+    cptc::dev_free(tmp);
     return rc;
 }
 

@@ -16,10 +16,12 @@
 #include <cstdlib>
 #include <cstring>
 #include <numeric>
+#include <optional>
 #include <random>
 #include <string>
 #include <vector>
 
+#include "dev_pool.hpp"
 #include "hip_util.hpp"
 #include "host_util.hpp"
 #include "layout_nd.hpp"
@@ -301,14 +303,13 @@ int dmalloc(T** p, size_t n)
 {
     *p = nullptr;
     if (n == 0) return CPTC_OK;
-    CPTC_HIP(hipMalloc(reinterpret_cast<void**>(p), n * sizeof(T)));
-    return CPTC_OK;
+    return cptc::dev_alloc(p, n * sizeof(T));
 }
 
 template <class T>
 void dfree(T*& p)
 {
-    if (p) (void)hipFree(p);
+    cptc::dev_free(p);
     p = nullptr;
 }
 
@@ -387,6 +388,7 @@ struct Gen
     ~Gen()
     {
         if (s) (void)hipStreamSynchronize(s);
+        cptc::PoolScope scope(nullptr, true);   // nothing is queued on the blocks any more
         dfree(d_coords);
         dfree(d_vals);
         for (auto& p : d_F) dfree(p);
@@ -414,9 +416,9 @@ struct Gen
         dfree(d_L);
         dfree(d_usum);
         dfree(d_uimg64);
-        if (d_Fo) (void)hipFree(d_Fo);
-        if (d_us_order) (void)hipFree(d_us_order);
-        if (d_us_chunk) (void)hipFree(d_us_chunk);
+        dfree(d_Fo);
+        dfree(d_us_order);
+        dfree(d_us_chunk);
         if (s) (void)hipStreamDestroy(s);
     }
 
@@ -732,8 +734,8 @@ int build_unit_groups(const cptc::DevUnitsN& u, int R, hipStream_t s, uint32_t* 
     for (int q = 0; q < 3; ++q)
     {
         CPTC_TRY(cptc_dense_groups(hdr.data(), 6, nu, q, cap, ord.data(), off.data(), &ng[q]));
-        CPTC_HIP(hipMalloc(&order[q], nu * sizeof(uint32_t)));
-        CPTC_HIP(hipMalloc(&goff[q], (ng[q] + 1) * sizeof(uint32_t)));
+        CPTC_TRY(cptc::dev_alloc(&order[q], nu * sizeof(uint32_t)));
+        CPTC_TRY(cptc::dev_alloc(&goff[q], (ng[q] + 1) * sizeof(uint32_t)));
         CPTC_HIP(hipMemcpyAsync(order[q], ord.data(), nu * sizeof(uint32_t), hipMemcpyHostToDevice, s));
         CPTC_HIP(hipMemcpyAsync(goff[q], off.data(), (ng[q] + 1) * sizeof(uint32_t),
                                 hipMemcpyHostToDevice, s));
@@ -754,8 +756,8 @@ int build_unit_sums_plan(const cptc::DevUnitsN& u, hipStream_t s, uint32_t*& d_o
                             hipMemcpyDeviceToHost, s));
     CPTC_HIP(hipStreamSynchronize(s));
     CPTC_TRY(cptc_gen_unit_sums_plan(hdr.data(), nu, 8, ord.data(), off.data(), &nchunks));
-    CPTC_HIP(hipMalloc(&d_order, nu * sizeof(uint32_t)));
-    CPTC_HIP(hipMalloc(&d_chunk, (nchunks + 1) * sizeof(uint32_t)));
+    CPTC_TRY(cptc::dev_alloc(&d_order, nu * sizeof(uint32_t)));
+    CPTC_TRY(cptc::dev_alloc(&d_chunk, (nchunks + 1) * sizeof(uint32_t)));
     CPTC_HIP(hipMemcpyAsync(d_order, ord.data(), nu * sizeof(uint32_t), hipMemcpyHostToDevice, s));
     CPTC_HIP(hipMemcpyAsync(d_chunk, off.data(), (nchunks + 1) * sizeof(uint32_t),
                             hipMemcpyHostToDevice, s));
@@ -865,7 +867,9 @@ extern "C" int cptc_gen_create(const cptc_coo* coo, const cptc_gen_opts* opts, v
                      "cptc_gen_create: dim %d = %llu", m, (unsigned long long)coo->dims[m]);
     CPTC_TRY(check_indices(coo));
     auto* g = new Gen();
+    std::optional<cptc::PoolScope> scope;   // ends before g's stream does
     auto fail = [&](int rc) {
+        scope.reset();
         delete g;
         return rc;
     };
@@ -901,6 +905,7 @@ extern "C" int cptc_gen_create(const cptc_coo* coo, const cptc_gen_opts* opts, v
 
     GEN_HIP(hipStreamCreateWithFlags(&g->s, hipStreamNonBlocking));
     hipStream_t s = g->s;
+    scope.emplace(s);   // the set-up's blocks: everything below runs on s
     const size_t RR = size_t(R) * R;
     const uint64_t ncoords = uint64_t(N) * g->nnz;
     GEN_TRY(dmalloc(&g->d_coords, ncoords));
@@ -1006,16 +1011,17 @@ extern "C" int cptc_gen_create(const cptc_coo* coo, const cptc_gen_opts* opts, v
                 }
                 std::vector<const double*> fo;
                 for (int o : g->units.outer) fo.push_back(g->d_F[o]);
-                GEN_HIP(hipMalloc(&g->d_Fo, fo.size() * sizeof(double*)));
-                GEN_HIP(hipMemcpy(g->d_Fo, fo.data(), fo.size() * sizeof(double*),
-                                  hipMemcpyHostToDevice));
+                GEN_TRY(cptc::dev_alloc(&g->d_Fo, fo.size() * sizeof(double*)));
+                GEN_HIP(hipMemcpyAsync(g->d_Fo, fo.data(), fo.size() * sizeof(double*),
+                                       hipMemcpyHostToDevice, s));
+                GEN_HIP(hipStreamSynchronize(s));
                 g->unit_sums = true;
             }
             if (g->tile_b3)
             {
                 const uint64_t md = std::max({g->dims[in[0]], g->dims[in[1]], g->dims[in[2]]});
                 g->tile_ws_bytes = cptc_tile_operands_bytes(md, R);
-                GEN_HIP(hipMalloc(&g->d_tile_ws, g->tile_ws_bytes));
+                GEN_TRY(cptc::dev_alloc(&g->d_tile_ws, g->tile_ws_bytes));
                 // compacted split unit images, one per inner slot (the order-3
                 // tiles' format)
                 const char* ce = std::getenv("GEN_TILE_COMPACT");

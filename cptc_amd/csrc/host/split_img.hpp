@@ -9,6 +9,7 @@
 #include <cstdint>
 
 #include "cptc_hip.h"
+#include "dev_pool.hpp"
 #include "hip_util.hpp"
 
 namespace cptc {
@@ -25,7 +26,7 @@ struct SplitImg
 inline void free_split_img(SplitImg& g)
 {
     for (void* p : {static_cast<void*>(g.cmask), static_cast<void*>(g.segoff), g.seg})
-        if (p) (void)hipFree(p);
+        dev_free(p);
     g = SplitImg{};
 }
 
@@ -44,11 +45,11 @@ inline int build_split_img(const float* tiles, size_t nt, int slot, SplitImg& g,
             if (!ok) free_split_img(g);
         }
     } guard{g};
-    CPTC_HIP(hipMalloc(&g.cmask, nt * 64 * sizeof(uint32_t)));
-    CPTC_HIP(hipMalloc(&g.segoff, (nt + 1) * sizeof(uint32_t)));
+    CPTC_TRY(dev_alloc(&g.cmask, nt * 64 * sizeof(uint32_t)));
+    CPTC_TRY(dev_alloc(&g.segoff, (nt + 1) * sizeof(uint32_t)));
     CPTC_TRY(cptc_dense_tiles_compact3_mask(tiles, nt, slot, g.cmask, g.segoff, &g.nseg, s));
     if (g.nseg * 16u >= 0xFFFFFFF0ull) return CPTC_OK;
-    CPTC_HIP(hipMalloc(&g.seg, std::max<uint64_t>(g.nseg, 1) * 16));
+    CPTC_TRY(dev_alloc(&g.seg, std::max<uint64_t>(g.nseg, 1) * 16));
     CPTC_TRY(cptc_dense_tiles_compact3_fill(tiles, nt, slot, g.cmask, g.segoff, g.seg, s));
     guard.ok = true;
     return CPTC_OK;

@@ -9,6 +9,7 @@
 #include <rocprim/device/device_run_length_encode.hpp>
 #include <rocprim/device/device_scan.hpp>
 
+#include "../host/dev_pool.hpp"
 #include "../host/hip_util.hpp"
 
 namespace cptc {
@@ -19,14 +20,13 @@ int dalloc(T** p, size_t n)
 {
     *p = nullptr;
     if (n == 0) return CPTC_OK;
-    CPTC_HIP(hipMalloc(reinterpret_cast<void**>(p), n * sizeof(T)));
-    return CPTC_OK;
+    return cptc::dev_alloc(p, n * sizeof(T));
 }
 
 template <class T>
 void dfree(T*& p)
 {
-    if (p) (void)hipFree(p);
+    cptc::dev_free(p);
     p = nullptr;
 }
 

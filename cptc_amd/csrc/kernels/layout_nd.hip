@@ -242,7 +242,7 @@ void free_view(DevViewN& v)
     dfree(v.d_start);
     dfree(v.d_cnt);
     dfree(v.d_single);
-    if (v.d_key) (void)hipFree(v.d_key);
+    dev_free(v.d_key);
     v.d_key = nullptr;
     v.key_bytes = 0;
     v.level_bits.clear();
@@ -421,6 +421,7 @@ int build_segments(const uint32_t* d_sorted_rows, uint64_t nnz, bool force_accum
     CPTC_TRY(upload(&out.d_start, start, s));
     CPTC_TRY(upload(&out.d_cnt, cnt, s));
     CPTC_TRY(upload(&out.d_single, single, s));
+    CPTC_HIP(hipStreamSynchronize(s));   // the vectors outlive their copies
     return CPTC_OK;
 }
 
@@ -499,7 +500,7 @@ int work_view_nd_device(int N, const uint64_t* dims, int n, const uint32_t* d_co
     out.key_bytes = cptc_level_key_bytes(nlev, out.level_bits.data());
     if (out.key_bytes > 0)
     {
-        CPTC_HIP(hipMalloc(&out.d_key, size_t(M) * size_t(out.key_bytes)));
+        CPTC_TRY(dev_alloc(&out.d_key, size_t(M) * size_t(out.key_bytes)));
         CPTC_TRY(cptc_pack_level_keys(nlev, out.d_sc, M, out.level_bits.data(), out.d_key,
                                       out.key_bytes, s));
     }

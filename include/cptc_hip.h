@@ -73,6 +73,9 @@ int cptc_dev_download(void* dst, const void* d_src, size_t bytes);
 int cptc_dev_memset(void* d_ptr, int value, size_t bytes);
 /* hipDeviceSynchronize, reporting any pending asynchronous error. */
 int cptc_dev_sync(void);
+/* Gives back the device blocks (at most 1 GiB) that the library keeps from
+ * destroyed cptc_als3_* / cptc_gen_* handles for the next one's set-up. */
+int cptc_dev_trim(void);
 
 /* ========================================================================
  * Ingest.

@@ -661,3 +661,73 @@ def test_cli_profile_line(ca, dev, tmp_path):
         parts = vals["gram"] + vals["mttkrp"] + vals["solve"] + vals["fit"]
         assert parts <= vals["iter"] * 1.0001 + 1e-3, vals
         assert lines[lines.index(l) - 1].startswith(f"[ALS] iter {k + 1}/3 ")
+
+
+def test_setup_blocks_reused(ca, dev):
+    """The set-up's device blocks pass from one handle to the next: layouts,
+    factors and MTTKRPs of tensors of several sizes are the same with fresh
+    blocks (after cptc_dev_trim), with blocks of other handles, while another
+    handle lives and from two threads in turn.  MTTKRPs (atomic adds) within
+    1e-13, the rest exactly."""
+    import threading
+
+    ts = [ca.synth_zipf((700, 400, 1500), (1.1, 1.1, 1.1), 120000, 0, 3),
+          clustered(ca, 4),
+          ca.synth_zipf((90, 50, 70), (0.5, 0.5, 0.5), 9000, 0, 5)]
+    t4 = ca.synth_zipf((40, 24, 70, 90), (0.0, 0.0, 1.2, 1.2), 60000, 2, 6)
+
+    def look(t, R=12):
+        with ca.Als3(t, R=R, path=2) as h:
+            w = 2 if h.info.fp64_merged else 0
+            out = [h.view(w, m)[k] for m in range(3)
+                   for k in ("coords", "vals", "blk_row", "blk_start", "blk_cnt")]
+            out += [h.factor(m, unpermuted=True) for m in range(3)]
+            return out, [h.mttkrp(m) for m in range(3)]
+
+    def look4():
+        with ca.Gen(t4, R=8) as g:
+            out = [g.coords()] + [g.factor(m) for m in range(4)]
+            return out, [g.mttkrp(m) for m in range(4)]
+
+    def same(a, b):
+        assert all(np.array_equal(x, y) for x, y in zip(a[0], b[0]))
+        assert all(rel_err(x, y) < 1e-13 for x, y in zip(a[1], b[1]))
+
+    ref = []
+    for t in ts:
+        assert ca.lib.cptc_dev_trim() == 0
+        ref.append(look(t))
+    assert ca.lib.cptc_dev_trim() == 0
+    ref4 = look4()
+    for _ in range(2):
+        for t, r in zip(ts, ref):
+            same(look(t), r)
+        same(look4(), ref4)
+    with ca.Als3(ts[0], R=12, path=2) as live:
+        before = [live.mttkrp(m) for m in range(3)]
+        for t, r in zip(ts, ref):
+            same(look(t), r)
+        assert all(rel_err(live.mttkrp(m), before[m]) < 1e-13 for m in range(3))
+    got, errs, one = [None, None], [], threading.Lock()
+
+    def turn(f, *a):   # one driver at a time on a device; the blocks change threads
+        with one:
+            return f(*a)
+
+    def work(q):
+        try:
+            got[q] = [turn(look, t) for t in ts] if q else [turn(look4) for _ in range(4)]
+        except Exception as e:   # noqa: BLE001  (reported by the main thread)
+            errs.append(e)
+
+    th = [threading.Thread(target=work, args=(q,)) for q in range(2)]
+    for x in th:
+        x.start()
+    for x in th:
+        x.join()
+    assert not errs, errs
+    for g in got[0]:
+        same(g, ref4)
+    for g, r in zip(got[1], ref):
+        same(g, r)
+    assert ca.lib.cptc_dev_trim() == 0

@@ -115,8 +115,8 @@ struct Als3
     double* d_fit_hist = nullptr;
     size_t fit_hist_cap = 0;
     // quiet runs of launch-bound problems replay one captured iteration
-    // bit m: mode m's update is one launch (update3_small); bit 3:
-    // mode C's also forms the fit scalars and clears FtV for mode A
+    // bit m: mode m's update is update3_small; bit 3: mode C's also forms the
+    // fit scalars and clears FtV for mode A
     int small_upd = 0;
     int graph_mode = 0;                  // 1: replay untimed iterations (ALS_GRAPH / automatic)
     hipGraphExec_t gexec = nullptr;      // the captured steady-state iteration
@@ -323,20 +323,21 @@ void choose_graph(Als3& h)
     else h.graph_mode = double(h.nnz) * double(h.R) < double(1u << 30) ? 1 : 0;
 }
 
-// Small factors (R <= 32, at most UPDATE3_SMALL_MAX_ROWS rows): a mode's
-// apply, Gram, norms, normalisation, scaling and the next mode's FtF in one
-// launch instead of five, and mode C's with the Gram fit and the
-// clearing of FtV for mode A (two launches fewer again).  Config 1 (256^3,
-// R = 32): 0.198 ms per iteration with the separate launches.  The ALS_DEBUG
-// dump reads mode C's MTTKRP after the iteration, so it keeps the separate
-// fit.  ALS_SMALL_UPDATE=0 keeps the separate launches.
+// R <= 32: a mode's apply, Gram, norms, normalisation, scaling, the next
+// mode's FtF and its pseudoinverse in one launch (up to 256 rows) or three
+// instead of six, and mode C's with the Gram fit and the clearing of FtV for
+// mode A (two launches fewer again).  256^3, R = 32: 0.198 ms per iteration
+// with the separate launches, 0.151 with one; 9000 x 5003 x 28000 at R = 25
+// 0.380 ms with the separate ones, 0.343 with three.  The ALS_DEBUG dump
+// reads mode C's MTTKRP after the iteration, so it keeps the separate fit.
+// ALS_SMALL_UPDATE=0 keeps the separate launches.
 void choose_small_update(Als3& h)
 {
     h.small_upd = 0;
     const char* e = std::getenv("ALS_SMALL_UPDATE");
     if ((e && std::strcmp(e, "0") == 0) || h.R > 32) return;
     for (int m = 0; m < 3; ++m)
-        if (h.dims[m] >= 1 && h.dims[m] <= UPDATE3_SMALL_MAX_ROWS) h.small_upd |= 1 << m;
+        if (h.dims[m] >= 1) h.small_upd |= 1 << m;
     if ((h.small_upd & 4) && !(h.o.verbose && std::getenv("ALS_DEBUG"))) h.small_upd |= 8;
 }
 
@@ -686,8 +687,8 @@ int update_mode(Als3& h, int mode, double* d_fit = nullptr, bool* fit_done = nul
     const int next = (mode + 1) % 3, other = 3 - next - mode;
     if (h.small_upd & (1 << mode))
     {
-        // one launch: apply, Gram, norms, normalisation, scaling, the next
-        // FtF, the next MTTKRP's cleared FtV and, for mode C, the fit
+        // apply, Gram, norms, normalisation, scaling, the next FtF and its
+        // pinv, the next MTTKRP's cleared FtV and, for mode C, the fit
         const bool fuse = h.gram_ok[other];
         const bool fit = mode == 2 && d_fit && (h.small_upd & 8);
         const size_t nz = (mode < 2 || fit) ? h.dims[next] * size_t(R) : 0;
@@ -1167,7 +1168,11 @@ extern "C" int cptc_als3_info_get(void* handle, cptc_als3_info* info)
     info->graph_captures = h->n_captures;
     info->fp64_merged = h->aviews.ready ? 1 : 0;
     for (int m = 0; m < 3; ++m) info->merged_segments[m] = h->aviews.ready ? h->aviews.nseg[m] : 0;
+    // the modes within cptc_update_small3's own limit
     info->small_update = h->small_upd;
+    for (int m = 0; m < 3; ++m)
+        if (h->dims[m] > cptc::UPDATE3_SMALL_MAX_ROWS)
+            info->small_update &= m == 2 ? 3 : ~(1 << m);
     info->tiles_beside = (h->dense_beside && h->use_mfma && h->part.ntiles > 0 && !h->fused) ? 1 : 0;
     return CPTC_OK;
 }

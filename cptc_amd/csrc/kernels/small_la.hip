@@ -1316,9 +1316,9 @@ int scale_launch(double* F, size_t rows, int R, const double* norms, const cptc:
 }
 
 // ---------------------------------------------------------------------------
-// A small factor's whole update in one launch (rows <= UPD3_MAX_ROWS, R <=
-// 16 NT <= 32) on the FP64 matrix cores (v_mfma_f64_16x16x4f64), the six
-// launches of apply + Gram + norms + scaling (+ fit) in one:
+// A mode's whole update at R <= 16 NT <= 32 on the FP64 matrix cores
+// (v_mfma_f64_16x16x4f64), in place of the launches of apply + Gram + norms +
+// scaling + pinv (+ fit):
 //   F = (FtV Ainv) / lambda                      (apply_small_kernel)
 //   G = F^T F; n_r = sqrt(G_rr); lambda_r *= n_r, 0 when n_r < 1e-14;
 //   G_rs /= n_r n_s (0 at a tiny norm); FtF = G .* other when other is given
@@ -1327,22 +1327,27 @@ int scale_launch(double* F, size_t rows, int R, const double* norms, const cptc:
 // With fit_out (the iteration's last mode), also the Gram fit scalars of
 // fit_finalize_kernel: fit_out[0] = sum_r lambda_r <F[:, r], FtV[:, r]>,
 // fit_out[1] = sum_{r,s} lambda_r lambda_s G_0 G_1 G_2 [r][s] (grams holds
-// G_0 and G_1; G_2 is this launch's G).  Last, Z[0, nz) is cleared (Z is
-// FtV).
-// Stage 1, every workgroup: wave w takes the 16-row block 4 blockIdx + w
-// (and every 4 gridDim-th after it); the apply's accumulator element v of
-// lane l is F[16 b + l / 16 + 4 v][16 t + l % 16], stored unscaled, and it
-// is also the Gram's A operand (F^T, ranks 16 t .. + 15 against rows 16 b +
-// 4 v .. + 3) and B operand, so the Gram partial needs no data movement;
-// the workgroup's Gram (and, for the fit, per-rank <F, FtV>) partial goes
-// to part[blockIdx] after the four waves' sums in wave order.  Stage 2, the
-// workgroup that finishes last (a device counter taken after a release
-// fence; no workgroup waits for another): the partials in workgroup order,
-// the norms, lambda, G, FtF and the fit, then the factor scaled in place
-// and FtV cleared (every workgroup's reads of FtV precede its count).  The
-// last workgroup resets the counter, so launches on one device must not
-// overlap (the library's scratch buffers have the same rule).  The sums run
-// in the matrix cores' order, not the separate kernels'.
+// G_0 and G_1; G_2 is this launch's G).  Z[0, nz) is cleared (Z is FtV), and
+// with Anext the next mode's pinv(FtF) is formed.
+//
+// Three launches, any number of rows:
+//   parts: wave w takes the 16-row block 8 blockIdx + w (and every 8
+//     gridDim-th after it); the apply's accumulator element v of lane l is
+//     F[16 b + l / 16 + 4 v][16 t + l % 16], stored unscaled, and it is also
+//     the Gram's A operand (F^T, ranks 16 t .. + 15 against rows 16 b + 4 v
+//     .. + 3) and B operand, so the Gram partial needs no data movement; the
+//     workgroup's Gram (and, for the fit, per-rank <F, FtV>) partial goes to
+//     part[blockIdx] after the eight waves' sums in wave order;
+//   finish: one workgroup sums the partials in workgroup order and forms the
+//     norms, lambda, G, FtF and the fit;
+//   scale: the factor scaled in place and FtV cleared over the whole chip,
+//     the pinv in a workgroup of its own beside them.
+// The sums run in the matrix cores' order, not the separate kernels'.  Up to
+// 256 rows one workgroup does it all (update3_one_kernel, below).  The form
+// before, one launch whose last workgroup to finish summed, rescaled the
+// whole factor and formed the pinv, against these three, back to back: R = 25
+// 512 rows 21.1 / 20.2 us, 1000 27.1 / 21.0, 3001 57.4 / 23.7, 4096 73.8 /
+// 24.4; R = 32 at 4096 rows 82.9 / 26.5.
 // ---------------------------------------------------------------------------
 // Loads that may be padding are zeroed by an AND with a mask made opaque
 // by an empty asm, not by a select: the compiler turns `cond ? load : 0`
@@ -1365,33 +1370,38 @@ __device__ __forceinline__ double upd3_keep(double v)
     return v;
 }
 
-constexpr int UPD3_T = 256;
+constexpr int UPD3_T = 512;         // parts
+constexpr int UPD3_SCALE_T = 256;   // scale
 constexpr int UPD3_WAVES = UPD3_T / WAVE;
-constexpr int UPD3_MAX_ROWS = 4096;
-constexpr int UPD3_MAX_P = UPD3_MAX_ROWS / (16 * UPD3_WAVES);   // 64 workgroups
-__device__ unsigned int upd3_count;   // zero at load; the last workgroup resets it
+// workgroups of the parts launch: one 16-row block a wave up to 4096 rows,
+// and no more than 32 partials to sum until the waves have two blocks each
+// (a partial costs the one workgroup that sums them ~0.13 us)
+constexpr int UPD3_P = 32, UPD3_MAX_P = 64;
+constexpr size_t UPD3_WIDE_ROWS = 8192;
+
+
+// The parts launch's work: this workgroup's row blocks of F, unscaled, and its
+// Gram (and fit) partial to part[blockIdx].
+template <int NT>
+struct Upd3Lds
+{
+    static constexpr int NP = NT * (NT + 1) / 2;   // tile pairs (a <= c) of the Gram
+    double gl[UPD3_WAVES][NP][256];
+    double fit_s[UPD3_WAVES][32];
+};
 
 template <int NT>
-__global__ __launch_bounds__(UPD3_T) void update3_small_kernel(
-    const double* Y, const double* __restrict__ Ainv, double* F, int rows, int R,
-    double* __restrict__ G, double* __restrict__ norms, double* lambda,
-    const double* __restrict__ other, double* __restrict__ FtF, double* Z, int nz,
-    const double* __restrict__ grams, double* __restrict__ fit_out, double* part,
-    double* __restrict__ Anext, double* __restrict__ Vw)
+__device__ __forceinline__ void upd3_stage1(const double* Y, const double* __restrict__ Ainv,
+                                            double* F, int rows, int R, const double* lambda,
+                                            bool fit, double* part, Upd3Lds<NT>& sm)
 {
-    constexpr int NP = NT * (NT + 1) / 2;   // tile pairs (a <= c) of the Gram
+    constexpr int NP = Upd3Lds<NT>::NP;
     constexpr int KS = 4 * NT;              // K steps of 4 over R padded to 16 NT
-    __shared__ double gl[UPD3_WAVES][NP][256];
-    __shared__ double g_s[32][33], f_s[32][33];
-    __shared__ double n_s[32], lamn_s[32], fit_s[UPD3_WAVES][32], fs_s[32];
-    __shared__ double red2[UPD3_WAVES];
-    __shared__ int last_s, decl_s;
     const int tid = threadIdx.x, w = tid / WAVE, l = tid % WAVE;
     const int lr = l % 16, lk = l / 16;
     const int RR = R * R;
     const int P = int(gridDim.x);
     const int stride = R * (R + 1);   // one partial: RR Gram entries, then R fit sums
-    // ---- stage 1 -------------------------------------------------------
     double bop[KS][NT];
 #pragma unroll
     for (int kk = 0; kk < KS; ++kk)
@@ -1426,7 +1436,7 @@ __global__ __launch_bounds__(UPD3_T) void update3_small_kernel(
                                upd3_mask(row0 + lr < rows && k < R));
         }
         // the fit's FtV entries at the accumulator's positions (loaded on
-        // every path, pinned after the products; used only with fit_out)
+        // every path, pinned after the products; used only with fit)
         double ym[NT][4];
 #pragma unroll
         for (int t = 0; t < NT; ++t)
@@ -1452,7 +1462,7 @@ __global__ __launch_bounds__(UPD3_T) void update3_small_kernel(
                 f[t][v] = x;
                 if (in) F[size_t(row) * R + c] = x;
                 const double y = upd3_keep(ym[t][v]);
-                if (fit_out) sp[t] += in ? x * y : 0.0;
+                if (fit) sp[t] += in ? x * y : 0.0;
             }
         }
         int p = 0;
@@ -1470,14 +1480,14 @@ __global__ __launch_bounds__(UPD3_T) void update3_small_kernel(
 #pragma unroll
     for (int p = 0; p < NP; ++p)
 #pragma unroll
-        for (int v = 0; v < 4; ++v) gl[w][p][(lk + 4 * v) * 16 + lr] = gacc[p][v];
-    if (fit_out)
+        for (int v = 0; v < 4; ++v) sm.gl[w][p][(lk + 4 * v) * 16 + lr] = gacc[p][v];
+    if (fit)
 #pragma unroll
         for (int t = 0; t < NT; ++t)
         {
             sp[t] += __shfl_xor(sp[t], 16);
             sp[t] += __shfl_xor(sp[t], 32);
-            if (lk == 0) fit_s[w][16 * t + lr] = sp[t];
+            if (lk == 0) sm.fit_s[w][16 * t + lr] = sp[t];
         }
     __syncthreads();
     double* my = part + size_t(blockIdx.x) * stride;
@@ -1487,7 +1497,7 @@ __global__ __launch_bounds__(UPD3_T) void update3_small_kernel(
         const int a = (p == 2) ? 1 : 0, c = (p == 0) ? 0 : 1;
         double s = 0.0;
 #pragma unroll
-        for (int q = 0; q < UPD3_WAVES; ++q) s += gl[q][p][e];
+        for (int q = 0; q < UPD3_WAVES; ++q) s += sm.gl[q][p][e];
         const int i = 16 * a + m, j = 16 * c + n;
         if ((a != c || m <= n) && i < R && j < R)
         {
@@ -1495,194 +1505,143 @@ __global__ __launch_bounds__(UPD3_T) void update3_small_kernel(
             my[j * R + i] = s;
         }
     }
-    if (fit_out && tid < R)
+    if (fit && tid < R)
     {
         double s = 0.0;
 #pragma unroll
-        for (int q = 0; q < UPD3_WAVES; ++q) s += fit_s[q][tid];
+        for (int q = 0; q < UPD3_WAVES; ++q) s += sm.fit_s[q][tid];
         my[RR + tid] = s;
     }
-    // every thread's stores (factor and partial) visible device-wide, then
-    // one count per workgroup
-    __threadfence();
-    __syncthreads();
-    if (tid == 0) last_s = (atomicAdd(&upd3_count, 1u) == unsigned(P - 1)) ? 1 : 0;
-    __syncthreads();
-    if (!last_s) return;
-    // ---- stage 2: the last workgroup --------------------------------------
-    __threadfence();   // acquire: the other workgroups' stores are seen
-    // every load that does not depend on the sums is issued first: the
-    // factor's first SB entries of this thread's column (scaling thread t:
-    // column t % R, rows t / R + k rpp; with Anext wave 0 runs the sweep
-    // instead and waves 1.. scale), the next FtF's other Gram and the fit's
-    // two Grams (entries tid + q T, RR <= 4 T)
-    constexpr int SB = 32;
-    const int nsc = Anext ? UPD3_T - WAVE : UPD3_T;
-    const int st = Anext ? tid - WAVE : tid;
-    const int stc = st < 0 ? 0 : st;
-    const int c0 = stc % R, rpp = nsc / R, r0 = stc / R;
-    double fv[SB];
+}
+
+template <int NT>
+__global__ __launch_bounds__(UPD3_T) void update3_parts_kernel(const double* Y,
+                                                               const double* __restrict__ Ainv,
+                                                               double* F, int rows, int R,
+                                                               const double* __restrict__ lambda,
+                                                               int fit, double* part)
+{
+    __shared__ Upd3Lds<NT> sm;
+    upd3_stage1<NT>(Y, Ainv, F, rows, R, lambda, fit != 0, part, sm);
+}
+
+// The P partials (R x R Gram entries, then R fit sums each) in workgroup
+// order; norms, lambda, the normalised G, FtF = G .* other and the fit
+// scalars.  R <= 32.
+// (in a fixed order, four sums over 16 loads in flight)
+__device__ __forceinline__ double upd3_sum(const double* __restrict__ part, int P, size_t stride)
+{
+    double t[4] = {0.0, 0.0, 0.0, 0.0};
+    int p = 0;
+    for (; p + 16 <= P; p += 16)
+    {
+        double v[16];
 #pragma unroll
-    for (int k = 0; k < SB; ++k) fv[k] = F[size_t(min(r0 + k * rpp, rows - 1)) * R + c0];
+        for (int k = 0; k < 16; ++k) v[k] = part[size_t(p + k) * stride];
+#pragma unroll
+        for (int k = 0; k < 16; ++k) t[k % 4] += v[k];
+    }
+    for (; p < P; p += 4)   // the rest; the last round reloads its own
+    {
+        double v[4];
+#pragma unroll
+        for (int k = 0; k < 4; ++k) v[k] = part[size_t(min(p + k, P - 1)) * stride];
+#pragma unroll
+        for (int k = 0; k < 4; ++k) t[k] += (p + k < P) ? v[k] : 0.0;
+    }
+    return (t[0] + t[1]) + (t[2] + t[3]);
+}
+
+__global__ __launch_bounds__(FIT_T) void update3_finish_kernel(
+    const double* __restrict__ part, int P, int R, double* __restrict__ G,
+    double* __restrict__ norms, double* __restrict__ lambda, const double* __restrict__ other,
+    double* __restrict__ FtF, const double* __restrict__ grams, double* __restrict__ fit_out)
+{
+    __shared__ double g_l[32 * 32], n_l[32], lam_l[32], red[FIT_T / WAVE];
+    const int RR = R * R, x = threadIdx.x, xc = min(x, RR - 1);
+    const size_t stride = size_t(R) * (R + 1);
     // (a null operand reads the partials instead: valid memory, unused)
-    const double* osrc = other ? other : part;
-    const double* gsrc = fit_out ? grams : part;
-    double ot[4], ga[4], gb[4];
-#pragma unroll
-    for (int q = 0; q < 4; ++q)
+    const double ot = (other ? other : part)[xc];
+    const double ga = (fit_out ? grams : part)[xc];
+    const double gb = (fit_out ? grams + RR : part)[xc];
+    const double lm = lambda[min(x, R - 1)];
+    const double g = upd3_sum(part + xc, P, stride);
+    if (x < RR) g_l[x] = g;
+    __syncthreads();
+    double ip = 0.0;
+    if (x < R)
     {
-        const int xc = min(tid + q * UPD3_T, RR - 1);
-        ot[q] = osrc[xc];
-        ga[q] = gsrc[xc];
-        gb[q] = gsrc[(fit_out ? size_t(RR) : 0) + xc];
-    }
-    // partial sums in workgroup order: the thread's Gram entries tid + q T
-    // (q < 4) and, for tid < R, the fit sum of rank tid; all loads of eight
-    // partials issued together
-    double gs[4] = {0.0, 0.0, 0.0, 0.0}, fsum = 0.0;
-    for (int q0 = 0; q0 < P; q0 += 8)
-    {
-        double v[8][5];
-#pragma unroll
-        for (int u = 0; u < 8; ++u)
+        const double n = sqrt(g_l[x * R + x]);
+        const double l = (n < 1e-14) ? 0.0 : lm * n;
+        n_l[x] = n;
+        lam_l[x] = l;
+        norms[x] = n;
+        lambda[x] = l;
+        if (fit_out)   // <F[:, r], FtV[:, r]> = <F_unscaled[:, r], FtV[:, r]> / n_r
         {
-            const double* pp = part + size_t(min(q0 + u, P - 1)) * stride;
-#pragma unroll
-            for (int q = 0; q < 4; ++q) v[u][q] = pp[min(tid + q * UPD3_T, RR - 1)];
-            v[u][4] = pp[RR + min(tid, R - 1)];
+            const double f = upd3_sum(part + RR + x, P, stride);
+            ip = l * ((n < 1e-14) ? 0.0 : f / n);
         }
-#pragma unroll
-        for (int u = 0; u < 8; ++u)
-            if (q0 + u < P)
-            {
-#pragma unroll
-                for (int q = 0; q < 4; ++q) gs[q] += v[u][q];
-                fsum += fit_out ? v[u][4] : 0.0;
-            }
-    }
-#pragma unroll
-    for (int q = 0; q < 4; ++q)
-    {
-        const int x = tid + q * UPD3_T;
-        if (x < RR) g_s[x / R][x % R] = gs[q];
-    }
-    // the early loads, issued before the partials', have landed: pin them here
-#pragma unroll
-    for (int k = 0; k < SB; ++k) fv[k] = upd3_keep(fv[k]);
-#pragma unroll
-    for (int q = 0; q < 4; ++q)
-    {
-        ot[q] = upd3_keep(ot[q]);
-        ga[q] = upd3_keep(ga[q]);
-        gb[q] = upd3_keep(gb[q]);
     }
     __syncthreads();
-    if (tid < R)
+    double md = 0.0;
+    if (x < RR)
     {
-        const double n = sqrt(g_s[tid][tid]);
-        n_s[tid] = n;
-        norms[tid] = n;
-        const double lm = (n < 1e-14) ? 0.0 : lambda[tid] * n;
-        lamn_s[tid] = lm;
-        lambda[tid] = lm;
+        const int i = x / R, j = x % R;
+        const double ni = n_l[i], nj = n_l[j];
+        const double v = (ni < 1e-14 || nj < 1e-14) ? 0.0 : g / (ni * nj);
+        G[x] = v;
+        if (other) FtF[x] = v * ot;
+        md = lam_l[i] * lam_l[j] * ga * gb * v;
     }
-    __syncthreads();
-#pragma unroll
-    for (int q = 0; q < 4; ++q)
+    if (fit_out)   // uniform
     {
-        const int x = tid + q * UPD3_T;
-        if (x < RR)
+        const double a = block_sum_all<FIT_T>(ip, red);
+        const double b = block_sum_all<FIT_T>(md, red);
+        if (x == 0)
         {
-            const int i = x / R, j = x % R;
-            const double ni = n_s[i], nj = n_s[j];
-            const double v = (ni < 1e-14 || nj < 1e-14) ? 0.0 : g_s[i][j] / (ni * nj);
-            g_s[i][j] = v;   // each entry read and written by its own thread only
-            G[x] = v;
-            if (other)
-            {
-                const double h = v * ot[q];
-                FtF[x] = h;
-                f_s[i][j] = h;
-            }
+            fit_out[0] = a;
+            fit_out[1] = b;
         }
     }
-    if (fit_out)   // uniform (a kernel argument)
+}
+
+// Workgroup 0: Anext = pinv(FtF) (when given); the others: F[:, r] /= n_r (0
+// at a tiny norm) and Z[0, nz) = 0.
+template <int NT>
+__global__ __launch_bounds__(UPD3_SCALE_T) void update3_scale_kernel(
+    double* __restrict__ F, size_t rows, int R, const double* __restrict__ norms, double* Z,
+    size_t nz, const double* __restrict__ FtF, double* __restrict__ Anext, double* __restrict__ Vw)
+{
+    __shared__ double jA[256 * NT * NT];   // the Jacobi path's A
+    __shared__ double n_l[32];
+    __shared__ int okp;
+    const int tid = threadIdx.x;
+    if (blockIdx.x == 0)
     {
-        // <F[:, r], FtV[:, r]> = <F_unscaled[:, r], FtV[:, r]> / n_r for the
-        // fit wave, and this thread's share of model^2, per wave
-        if (tid < R) fs_s[tid] = (n_s[tid] < 1e-14) ? 0.0 : fsum / n_s[tid];
-        double md = 0.0;
-#pragma unroll
-        for (int q = 0; q < 4; ++q)
+        if (!Anext) return;
+        if (tid < WAVE)
         {
-            const int x = tid + q * UPD3_T;
-            if (x < RR)
-            {
-                const int i = x / R, j = x % R;
-                md += lamn_s[i] * lamn_s[j] * ga[q] * gb[q] * g_s[i][j];
-            }
+            const int ok = sweep_wave<NT>(FtF, R, R, Anext);
+            if (tid == 0) okp = ok;
         }
-#pragma unroll
-        for (int o = WAVE / 2; o >= 1; o >>= 1) md += __shfl_xor(md, o);
-        if (l == 0) red2[w] = md;
-    }
-    __syncthreads();   // FtF in f_s; the fit's sums
-    if (st < 0)
-    {
-        // wave 0: the next mode's pinv (one-wave sweep)
-        const int okp = sweep_wave<NT>(&f_s[0][0], 33, R, Anext);
-        if (l == 0) decl_s = !okp;
-    }
-    else
-    {
-        if (fit_out && w == 1)
-        {
-            double ip = (l < R) ? lamn_s[l] * fs_s[l] : 0.0;
-#pragma unroll
-            for (int o = WAVE / 2; o >= 1; o >>= 1) ip += __shfl_xor(ip, o);
-            if (l == 0)
-            {
-                double m2 = 0.0;
-#pragma unroll
-                for (int q = 0; q < UPD3_WAVES; ++q) m2 += red2[q];
-                fit_out[0] = ip;
-                fit_out[1] = m2;
-            }
-        }
-        // the factor scaled in place, SB rows of the thread's column at a time
-        if (r0 < rpp)
-        {
-            const double n = n_s[c0];
-            const bool zero = n < 1e-14;
-#pragma unroll
-            for (int k = 0; k < SB; ++k)
-            {
-                const int i = r0 + k * rpp;
-                if (i < rows) F[size_t(i) * R + c0] = zero ? 0.0 : fv[k] / n;
-            }
-            for (int i0 = r0 + SB * rpp; i0 < rows; i0 += SB * rpp)
-            {
-#pragma unroll
-                for (int k = 0; k < SB; ++k)
-                    fv[k] = F[size_t(min(i0 + k * rpp, rows - 1)) * R + c0];
-#pragma unroll
-                for (int k = 0; k < SB; ++k)
-                {
-                    const int i = i0 + k * rpp;
-                    if (i < rows) F[size_t(i) * R + c0] = zero ? 0.0 : fv[k] / n;
-                }
-            }
-        }
-        for (int x = st; x < nz; x += nsc) Z[x] = 0.0;
-    }
-    if (Anext)   // uniform (a kernel argument)
-    {
         __syncthreads();
-        // a declined sweep: the Jacobi pseudoinverse of FtF by the whole
-        // workgroup (A in the Gram tiles' LDS, V in global scratch)
-        if (decl_s) jacobi_pinv_body<UPD3_T>(FtF, R, nullptr, Vw, Anext, 1, &gl[0][0][0]);
+        if (!okp) jacobi_pinv_body<UPD3_SCALE_T>(FtF, R, nullptr, Vw, Anext, 1, jA);
+        return;
     }
-    if (tid == 0) upd3_count = 0u;
+    if (tid < R) n_l[tid] = norms[tid];
+    __syncthreads();
+    const size_t total = rows * size_t(R), n = total > nz ? total : nz;
+    for (size_t x = size_t(blockIdx.x - 1) * UPD3_SCALE_T + tid; x < n;
+         x += size_t(gridDim.x - 1) * UPD3_SCALE_T)
+    {
+        if (x < total)
+        {
+            const double nr = n_l[x % size_t(R)];
+            F[x] = (nr < 1e-14) ? 0.0 : F[x] / nr;
+        }
+        if (x < nz) Z[x] = 0.0;
+    }
 }
 
 // The same update in one workgroup of UPD1_T threads for rows <= 16
@@ -2059,16 +2018,15 @@ int update3_small(double* d_FtV, double* d_Ainv, double* d_F, size_t rows, int R
                   size_t nzero, const double* d_grams, double* d_fit, int next_pinv,
                   hipStream_t s)
 {
-    CPTC_REQUIRE(R >= 1 && R <= 32 && rows >= 1 && rows <= UPDATE3_SMALL_MAX_ROWS,
-                 CPTC_ERR_ARG, "cptc_update_small3: rows %zu R %d (1..%zu rows, R <= 32)", rows,
-                 R, UPDATE3_SMALL_MAX_ROWS);
+    CPTC_REQUIRE(R >= 1 && R <= 32 && rows >= 1 && rows < (size_t(1) << 31), CPTC_ERR_ARG,
+                 "update3_small: rows %zu R %d", rows, R);
     CPTC_REQUIRE(d_FtV && d_Ainv && d_F && d_G && d_norms && d_lambda &&
                      (d_other == nullptr) == (d_FtF == nullptr) && (!d_fit || d_grams) &&
                      (!next_pinv || d_FtF) && nzero < (size_t(1) << 31),
                  CPTC_ERR_ARG, "cptc_update_small3: bad arguments");
-    static_assert(UPDATE3_SMALL_MAX_ROWS == size_t(UPD3_MAX_ROWS), "row limit");
-    const int nb = int((rows + 15) / 16);
-    const int P = (nb + UPD3_WAVES - 1) / UPD3_WAVES;   // one 16-row block per wave
+    const size_t nb = (rows + 15) / 16;
+    const int P = int(std::min<size_t>((nb + UPD3_WAVES - 1) / UPD3_WAVES,
+                                       rows > UPD3_WIDE_ROWS ? UPD3_MAX_P : UPD3_P));
     const size_t RR = size_t(R) * R;
     void* buf = nullptr;
     CPTC_TRY(cptc::scratch_get(cptc::SCR_GRAM, size_t(UPD3_MAX_P) * 32 * (32 + 1) * sizeof(double),
@@ -2084,10 +2042,10 @@ int update3_small(double* d_FtV, double* d_Ainv, double* d_F, size_t rows, int R
         Vw = static_cast<double*>(pb) + RR;
     }
     const int nr = int(rows), nz = int(nzero);
-    // one workgroup up to 256 rows, the multi-workgroup form above that
-    // (CPTC_UPD3_ONE_ROWS overrides the limit, at most 512; 0 = never).
-    // Per launch at R = 32: 256 rows 13.0 us in one workgroup against 15.0
-    // in four; 512 rows 22.0 us against 19.2 in eight.
+    // one workgroup up to 256 rows, three launches above that
+    // (CPTC_UPD3_ONE_ROWS overrides the limit, at most 512; 0 = never).  At R =
+    // 32, 256 rows take 13.0 us in one workgroup and 22 in three launches;
+    // 512 rows 22.0 in either.
     static const int one_rows = [] {
         const char* e = std::getenv("CPTC_UPD3_ONE_ROWS");
         return e ? std::atoi(e) : 256;
@@ -2105,14 +2063,16 @@ int update3_small(double* d_FtV, double* d_Ainv, double* d_F, size_t rows, int R
         CPTC_LAUNCHED();
         return CPTC_OK;
     }
-    if (R <= 16)
-        hipLaunchKernelGGL(update3_small_kernel<1>, dim3(P), dim3(UPD3_T), 0, s, d_FtV, d_Ainv,
-                           d_F, nr, R, d_G, d_norms, d_lambda, d_other, d_FtF, d_FtV, nz, d_grams,
-                           d_fit, part, Anext, Vw);
-    else
-        hipLaunchKernelGGL(update3_small_kernel<2>, dim3(P), dim3(UPD3_T), 0, s, d_FtV, d_Ainv,
-                           d_F, nr, R, d_G, d_norms, d_lambda, d_other, d_FtF, d_FtV, nz, d_grams,
-                           d_fit, part, Anext, Vw);
+    hipLaunchKernelGGL(R <= 16 ? update3_parts_kernel<1> : update3_parts_kernel<2>, dim3(P),
+                       dim3(UPD3_T), 0, s, d_FtV, d_Ainv, d_F, nr, R, d_lambda,
+                       int(d_fit != nullptr), part);
+    CPTC_LAUNCHED();
+    hipLaunchKernelGGL(update3_finish_kernel, dim3(1), dim3(FIT_T), 0, s, part, P, R, d_G, d_norms,
+                       d_lambda, d_other, d_FtF, d_grams, d_fit);
+    CPTC_LAUNCHED();
+    const unsigned grid = 1 + cptc::grid_for(std::max(rows * size_t(R), nzero), UPD3_SCALE_T, 2048);
+    hipLaunchKernelGGL(R <= 16 ? update3_scale_kernel<1> : update3_scale_kernel<2>, dim3(grid),
+                       dim3(UPD3_SCALE_T), 0, s, d_F, rows, R, d_norms, d_FtV, nzero, d_FtF, Anext, Vw);
     CPTC_LAUNCHED();
     return CPTC_OK;
 }
@@ -2125,6 +2085,9 @@ extern "C" int cptc_update_small3(double* d_FtV, double* d_Ainv, double* d_F, si
                                   const double* d_grams, double* d_fit, int next_pinv,
                                   void* stream)
 {
+    CPTC_REQUIRE(R >= 1 && R <= 32 && rows >= 1 && rows <= cptc::UPDATE3_SMALL_MAX_ROWS,
+                 CPTC_ERR_ARG, "cptc_update_small3: rows %zu R %d (1..%zu rows, R <= 32)", rows,
+                 R, cptc::UPDATE3_SMALL_MAX_ROWS);
     return cptc::update3_small(d_FtV, d_Ainv, d_F, rows, R, d_G, d_norms, d_lambda, d_other,
                                d_FtF, nzero, d_grams, d_fit, next_pinv, cptc::as_stream(stream));
 }

@@ -266,8 +266,8 @@ int cptc_gram_normalize_absorb_next(double* d_F, size_t rows, int R, double* d_G
                                     double* d_norms, double* d_lambda, const double* d_other,
                                     double* d_FtF, void* stream);
 
-/* One mode's whole update for a small factor in one launch (1 <= rows <=
- * 4096, R <= 32; FP64 matrix cores): F = (d_FtV * d_Ainv) /
+/* One mode's whole update for a small factor (1 <= rows <= 4096, R <= 32;
+ * FP64 matrix cores) in one launch up to 256 rows, in three above: F = (d_FtV * d_Ainv) /
  * lambda (cptc_apply_pinv's product with d_Ainv = pinv(FtF) given), then
  * cptc_gram_normalize_absorb_next on it (G, norms, lambda, F scaled, the
  * next FtF = G .* d_other when d_other / d_FtF are given), then
@@ -279,9 +279,9 @@ int cptc_gram_normalize_absorb_next(double* d_F, size_t rows, int R, double* d_G
  * cptc_pinv_sym of the new d_FtF (the same bits when the fast path accepts
  * it; the Jacobi pseudoinverse otherwise).  Results equal the separate
  * calls' up to summation order (als.cu:480-517, 659-715; solver.cu:900-1002).
- * Uses the library's Gram and pinv scratch and a device counter: calls that
- * overlap on one GPU race.  No reference counterpart: the reference runs
- * these as separate kernels. */
+ * Uses the library's Gram and pinv scratch: calls that overlap on one GPU
+ * race.  No reference counterpart: the reference runs these as separate
+ * kernels. */
 int cptc_update_small3(double* d_FtV, double* d_Ainv, double* d_F, size_t rows, int R,
                        double* d_G, double* d_norms, double* d_lambda, const double* d_other,
                        double* d_FtF, size_t nzero, const double* d_grams, double* d_fit,
@@ -508,9 +508,9 @@ typedef struct cptc_als3_info {
                                  one row-sorted view: one FP64 launch per mode, and the
                                  per-mode sparse kernel time covers every nonzero */
     uint64_t merged_segments[3];  /* segments of that view per mode (0: none) */
-    int small_update;         /* bit m: mode m's update runs as one launch
-                                 (cptc_update_small3; R <= 32, at most 4096 rows); bit 3:
-                                 mode C's launch also forms the Gram fit scalars */
+    int small_update;         /* bit m: mode m's update runs as cptc_update_small3 (R <= 32, at
+                                 most 4096 rows; larger factors take the same launches);
+                                 bit 3: mode C's also forms the Gram fit scalars */
 } cptc_als3_info;
 int cptc_als3_info_get(void* handle, cptc_als3_info* info);
 

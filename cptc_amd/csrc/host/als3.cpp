@@ -499,10 +499,7 @@ int create(const cptc_coo* coo, const cptc_als3_opts* opts, Als3* h)
     // every index must lie inside its mode (the device layout kernels index by it)
     for (int m = 0; m < 3; ++m)
     {
-        const uint32_t* c = coo->idx + size_t(m) * coo->nnz;
-        uint64_t mx = 0;
-        #pragma omp parallel for reduction(max : mx) schedule(static)
-        for (int64_t e = 0; e < int64_t(coo->nnz); ++e) mx = std::max<uint64_t>(mx, c[e]);
+        const uint64_t mx = cptc::max_u32(coo->idx + size_t(m) * coo->nnz, coo->nnz);
         CPTC_REQUIRE(coo->nnz == 0 || mx < h->dims[m], CPTC_ERR_ARG,
                      "cptc_als3_create: mode %d index %llu >= dim %llu", m,
                      (unsigned long long)mx, (unsigned long long)h->dims[m]);

@@ -275,9 +275,7 @@ int check_indices(const cptc_coo* c)
     for (int m = 0; m < c->nmodes; ++m)
     {
         const uint32_t* cm = c->idx + uint64_t(m) * c->nnz;
-        uint32_t mx = 0;
-#pragma omp parallel for reduction(max : mx)
-        for (int64_t e = 0; e < int64_t(c->nnz); ++e) mx = std::max(mx, cm[e]);
+        const uint32_t mx = cptc::max_u32(cm, c->nnz);
         CPTC_REQUIRE(c->nnz == 0 || uint64_t(mx) < c->dims[m], CPTC_ERR_ARG,
                      "coordinate %u of mode %d outside dim %llu", mx, m,
                      (unsigned long long)c->dims[m]);

@@ -28,6 +28,12 @@ inline uint64_t rng_u64(uint64_t seed, uint64_t stream, uint64_t ctr)
 // [0, 1) with 53 random bits.
 inline double u01(uint64_t x) { return double(x >> 11) * (1.0 / 9007199254740992.0); }
 
+// Largest of n values (0 for none).  One thread up to 4 M values (0.1 ms a
+// million): an OpenMP team keeps spinning for milliseconds after its loop, and
+// the set-up that follows shares the cores with it (1 M nonzeros: the rest of
+// a set-up took 1.9 ms longer).
+uint32_t max_u32(const uint32_t* v, size_t n);
+
 // Stable LSD radix sort of (key, payload) pairs on the low `key_bits` bits,
 // 11 bits per pass, OpenMP-parallel with per-thread histograms.
 template <class V>

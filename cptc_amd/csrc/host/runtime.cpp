@@ -9,6 +9,7 @@
 #include <vector>
 
 #include "hip_util.hpp"
+#include "host_util.hpp"
 
 namespace cptc {
 
@@ -52,6 +53,27 @@ void set_error(const char* fmt, ...)
     va_start(ap, fmt);
     std::vsnprintf(g_err, sizeof(g_err), fmt, ap);
     va_end(ap);
+}
+
+namespace {
+__attribute__((target_clones("avx2", "default"))) uint32_t max_serial(const uint32_t* v, size_t n)
+{
+    uint32_t mx = 0;
+    for (size_t e = 0; e < n; ++e) mx = v[e] > mx ? v[e] : mx;
+    return mx;
+}
+}  // namespace
+
+uint32_t max_u32(const uint32_t* v, size_t n)
+{
+    constexpr size_t PART = size_t(4) << 20;
+    if (n <= PART) return max_serial(v, n);
+    const int64_t parts = int64_t((n + PART - 1) / PART);
+    uint32_t mx = 0;
+    #pragma omp parallel for reduction(max : mx) schedule(static)
+    for (int64_t q = 0; q < parts; ++q)
+        mx = std::max(mx, max_serial(v + size_t(q) * PART, std::min(PART, n - size_t(q) * PART)));
+    return mx;
 }
 
 int scratch_get(int slot, size_t bytes, void** out)

@@ -42,7 +42,7 @@ __global__ __launch_bounds__(WAVE* WAVES) void mttkrp3_seg_kernel(
                                               blk_start, blk_cnt, F1, F2, FtV, R);
 }
 
-// R in (64, 128] with 16-byte rows: one element per wave (LPE = 64), so the
+// R > 64: one element per wave (LPE = 64), so the
 // window position, the element's coordinates and value, the run state and
 // the factor-row addresses are the same for every lane.  This variant keeps
 // them wave-uniform and spends as few issue slots per element as it can,
@@ -86,7 +86,10 @@ __global__ __launch_bounds__(WAVE* WAVES) __attribute__((amdgpu_waves_per_eu(1, 
     const int wave = __builtin_amdgcn_readfirstlane(tid / WAVE);
     const int r0 = int(blockIdx.y) * RT + lane * 2;
     const bool rank_ok = r0 < R;
-    const int rr = rank_ok ? r0 : 0;
+    // odd R: the last lane holds ranks R - 2 and R - 1 (in bounds), and only
+    // its second sum counts
+    const bool odd_last = r0 == R - 1;
+    const int rr = odd_last ? r0 - 1 : rank_ok ? r0 : 0;
     constexpr int sh0 = (MODE == 0) ? 15 : 30;
     constexpr int sh1 = (MODE == 2) ? 15 : 0;
     // factor rows by buffer loads: the row offset o*R*8 in soffset (scalar),
@@ -204,6 +207,7 @@ __global__ __launch_bounds__(WAVE* WAVES) __attribute__((amdgpu_waves_per_eu(1, 
         acc1 += t1 * f2.y;
     }
     if (!rank_ok) acc0 = acc1 = 0.0;
+    if (odd_last) acc0 = acc1;
 
     __shared__ double red[WAVES][RT];
     red[wave][lane * 2] = acc0;
@@ -220,7 +224,7 @@ __global__ __launch_bounds__(WAVE* WAVES) __attribute__((amdgpu_waves_per_eu(1, 
     }
 }
 
-// R <= 64 with 16-byte rows: EPW = 128 / RT element slots per wave (RT = 8,
+// R in [2, 64]: EPW = 128 / RT element slots per wave (RT = 8,
 // 16, 32, 64 -> 16, 8, 4, 2 slots of LPE = RT / 2 lanes), with the sum and
 // run logic of mttkrp3_seg_kernel; the per-element work is cut, because at
 // these R a lane's two ranks per element leave that kernel bound by
@@ -267,7 +271,10 @@ __global__ __launch_bounds__(WAVE* WAVES) void mttkrp3_seg_lanes_kernel(
     const int slot = lane / LPE;
     const int r0 = (lane % LPE) * 2;
     const bool rank_ok = r0 < R;
-    const uint32_t voff = uint32_t(rank_ok ? r0 : 0) * 8u;
+    // odd R: the element's last lane holds ranks R - 2 and R - 1 (in bounds),
+    // and only its second sum counts
+    const bool odd_last = r0 == R - 1;
+    const uint32_t voff = uint32_t(odd_last ? r0 - 1 : rank_ok ? r0 : 0) * 8u;
     constexpr int sh0 = (MODE == 0) ? 15 : 30;
     constexpr int sh1 = (MODE == 2) ? 15 : 0;
     const __amdgpu_buffer_rsrc_t rs1 =
@@ -383,6 +390,7 @@ __global__ __launch_bounds__(WAVE* WAVES) void mttkrp3_seg_lanes_kernel(
         acc1 += t1 * f2.y;
     }
     if (!rank_ok) acc0 = acc1 = 0.0;
+    if (odd_last) acc0 = acc1;
     // reduce the slots of the wave (lanes l, l ^ LPE, l ^ 2 LPE, ...)
 #pragma unroll
     for (int off = LPE; off < WAVE; off <<= 1)
@@ -408,49 +416,42 @@ __global__ __launch_bounds__(WAVE* WAVES) void mttkrp3_seg_lanes_kernel(
     }
 }
 
-template <int RT, int VEC>
+// A lane's two ranks are one 16-byte load, whatever the row's alignment (the
+// loads need 4 bytes): rows of odd R or on 8-byte bases split more lines but
+// keep the lane layout.  RT = 1 stands for R = 1, which has no second rank
+// to load beside the first.
+template <int RT>
 hipError_t launch_rt(int mode, const uint64_t* coords, const double* vals, const uint32_t* br,
                      const uint32_t* bs, const uint32_t* bc, size_t nblocks, const double* F1,
                      const double* F2, double* FtV, int R, hipStream_t s)
 {
     constexpr int WAVES = 4;
-    constexpr int UNROLL = CPTC_SPARSE3_UNROLL;
-    const unsigned ry = unsigned((R + RT - 1) / RT);
-    dim3 grid(unsigned(nblocks), ry);
-    // the wave-uniform kernel addresses rows by 32-bit byte offsets o * R * 8
-    // (o < 2^15), so it needs R * 8 * 2^15 < 2^31
-    if (RT <= 64 && VEC == 2)
+    const dim3 block(WAVE * WAVES);
+    auto go = [&](auto kern, unsigned ry) {
+        hipLaunchKernelGGL(kern, dim3(unsigned(nblocks), ry), block, 0, s, coords, vals, br, bs, bc,
+                           F1, F2, FtV, R);
+    };
+    if constexpr (RT > 1 && RT <= 64)
     {
-        constexpr int RL = RT <= 64 ? RT : 64;   // (the branch is dead for RT = 128)
-        constexpr int UL = CPTC_SPARSE3_LANES_UNROLL;
-        const dim3 block(WAVE * WAVES);
-        if (mode == 0)
-            hipLaunchKernelGGL((mttkrp3_seg_lanes_kernel<0, RL, WAVES, UL>), grid, block, 0, s,
-                               coords, vals, br, bs, bc, F1, F2, FtV, R);
-        else if (mode == 1)
-            hipLaunchKernelGGL((mttkrp3_seg_lanes_kernel<1, RL, WAVES, UL>), grid, block, 0, s,
-                               coords, vals, br, bs, bc, F1, F2, FtV, R);
-        else
-            hipLaunchKernelGGL((mttkrp3_seg_lanes_kernel<2, RL, WAVES, UL>), grid, block, 0, s,
-                               coords, vals, br, bs, bc, F1, F2, FtV, R);
+        constexpr int U = CPTC_SPARSE3_LANES_UNROLL;
+        if (mode == 0) go(mttkrp3_seg_lanes_kernel<0, RT, WAVES, U>, 1);
+        else if (mode == 1) go(mttkrp3_seg_lanes_kernel<1, RT, WAVES, U>, 1);
+        else go(mttkrp3_seg_lanes_kernel<2, RT, WAVES, U>, 1);
     }
-    else if (RT == 128 && VEC == 2 && R <= 8000)
+    else if (RT == 128 && R <= 8000)
     {
-        const dim3 block(WAVE * WAVES);
-        if (mode == 0)
-            hipLaunchKernelGGL((mttkrp3_seg_wave_kernel<0, WAVES, CPTC_SPARSE3_WAVE_UNROLL>), grid,
-                               block, 0, s, coords, vals, br, bs, bc, F1, F2, FtV, R);
-        else if (mode == 1)
-            hipLaunchKernelGGL((mttkrp3_seg_wave_kernel<1, WAVES, CPTC_SPARSE3_WAVE_UNROLL>), grid,
-                               block, 0, s, coords, vals, br, bs, bc, F1, F2, FtV, R);
-        else
-            hipLaunchKernelGGL((mttkrp3_seg_wave_kernel<2, WAVES, CPTC_SPARSE3_WAVE_UNROLL>), grid,
-                               block, 0, s, coords, vals, br, bs, bc, F1, F2, FtV, R);
+        // rows are addressed by 32-bit byte offsets o * R * 8 (o < 2^15), so
+        // this needs R * 8 * 2^15 < 2^31
+        constexpr int U = CPTC_SPARSE3_WAVE_UNROLL;
+        const unsigned ry = unsigned((R + 127) / 128);
+        if (mode == 0) go(mttkrp3_seg_wave_kernel<0, WAVES, U>, ry);
+        else if (mode == 1) go(mttkrp3_seg_wave_kernel<1, WAVES, U>, ry);
+        else go(mttkrp3_seg_wave_kernel<2, WAVES, U>, ry);
     }
     else
-        hipLaunchKernelGGL((mttkrp3_seg_kernel<RT, VEC, WAVES, UNROLL>), grid,
-                           dim3(WAVE * WAVES), 0, s, mode, coords, vals, br, bs, bc, F1, F2, FtV,
-                           R);
+        hipLaunchKernelGGL((mttkrp3_seg_kernel<RT == 1 ? 8 : 64, 1, WAVES, CPTC_SPARSE3_UNROLL>),
+                           dim3(unsigned(nblocks), unsigned((R + 63) / 64)), block, 0, s, mode,
+                           coords, vals, br, bs, bc, F1, F2, FtV, R);
     return hipGetLastError();
 }
 
@@ -518,43 +519,14 @@ extern "C" int cptc_mttkrp_sparse3(int mode, const uint64_t* d_coords, const dou
                      d_FtV,
                  CPTC_ERR_ARG, "cptc_mttkrp_sparse3: null pointer");
     hipStream_t s = cptc::as_stream(stream);
-    // 16-byte rows need an even R and 16-byte aligned factor bases.
-    const bool vec2 = (R % 2 == 0) && ((reinterpret_cast<uintptr_t>(d_F1) & 15) == 0) &&
-                      ((reinterpret_cast<uintptr_t>(d_F2) & 15) == 0);
-    hipError_t e;
-    if (vec2)
-    {
-        if (R <= 8)
-            e = launch_rt<8, 2>(mode, d_coords, d_vals, d_blk_row, d_blk_start, d_blk_cnt, nblocks,
+    auto launch = R == 1    ? launch_rt<1>
+                  : R <= 8  ? launch_rt<8>
+                  : R <= 16 ? launch_rt<16>
+                  : R <= 32 ? launch_rt<32>
+                  : R <= 64 ? launch_rt<64>
+                            : launch_rt<128>;
+    const hipError_t e = launch(mode, d_coords, d_vals, d_blk_row, d_blk_start, d_blk_cnt, nblocks,
                                 d_F1, d_F2, d_FtV, R, s);
-        else if (R <= 16)
-            e = launch_rt<16, 2>(mode, d_coords, d_vals, d_blk_row, d_blk_start, d_blk_cnt,
-                                 nblocks, d_F1, d_F2, d_FtV, R, s);
-        else if (R <= 32)
-            e = launch_rt<32, 2>(mode, d_coords, d_vals, d_blk_row, d_blk_start, d_blk_cnt,
-                                 nblocks, d_F1, d_F2, d_FtV, R, s);
-        else if (R <= 64)
-            e = launch_rt<64, 2>(mode, d_coords, d_vals, d_blk_row, d_blk_start, d_blk_cnt,
-                                 nblocks, d_F1, d_F2, d_FtV, R, s);
-        else
-            e = launch_rt<128, 2>(mode, d_coords, d_vals, d_blk_row, d_blk_start, d_blk_cnt,
-                                  nblocks, d_F1, d_F2, d_FtV, R, s);
-    }
-    else
-    {
-        if (R <= 8)
-            e = launch_rt<8, 1>(mode, d_coords, d_vals, d_blk_row, d_blk_start, d_blk_cnt, nblocks,
-                                d_F1, d_F2, d_FtV, R, s);
-        else if (R <= 16)
-            e = launch_rt<16, 1>(mode, d_coords, d_vals, d_blk_row, d_blk_start, d_blk_cnt,
-                                 nblocks, d_F1, d_F2, d_FtV, R, s);
-        else if (R <= 32)
-            e = launch_rt<32, 1>(mode, d_coords, d_vals, d_blk_row, d_blk_start, d_blk_cnt,
-                                 nblocks, d_F1, d_F2, d_FtV, R, s);
-        else
-            e = launch_rt<64, 1>(mode, d_coords, d_vals, d_blk_row, d_blk_start, d_blk_cnt,
-                                 nblocks, d_F1, d_F2, d_FtV, R, s);
-    }
     CPTC_REQUIRE(e == hipSuccess, CPTC_ERR_HIP, "cptc_mttkrp_sparse3 launch: %s",
                  hipGetErrorString(e));
     return CPTC_OK;

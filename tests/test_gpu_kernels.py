@@ -130,6 +130,34 @@ def test_sparse_mttkrp_misaligned_factor_base(ca, orc, dev):
     assert rel_err(out.numpy(), ref) <= 1e-10
 
 
+@pytest.mark.parametrize("R", [2, 3, 5, 7, 9, 15, 17, 25, 31, 33, 51, 63, 65, 99, 127, 129])
+def test_sparse_mttkrp_odd_ranks(ca, orc, dev, R):
+    """Odd R (rows on 8-byte boundaries, an element's last lane holding ranks R
+    - 2 and R - 1) and, at R = 2, one lane an element: every mode within
+    1e-10 of the oracle, with NaN before and after each factor, so that a
+    rank taken from beyond a row's or a factor's end shows."""
+    dims = (300, 200, 500)
+    t, views = zipf_views(ca, orc, dims, 40000, 60 + R, dup=True)
+    rng = np.random.default_rng(R)
+    F = [rng.standard_normal((d, R)) for d in dims]
+    nan = np.full(3, np.nan)
+    dF = [to_dev(ca, np.concatenate([nan, f.ravel(), nan])) for f in F]
+    at = [f.data_ptr() + 8 * len(nan) for f in dF]
+    for mode in range(3):
+        v = views[mode]
+        ref = orc.mttkrp3_view(views, mode, F[0].ravel(), F[1].ravel(), F[2].ravel(), R,
+                               dims[mode]).reshape(dims[mode], R)
+        dc, dv = to_dev(ca, v["coords"]), to_dev(ca, v["vals"])
+        br, bs, bc = (to_dev(ca, v[k]) for k in ("blk_row", "blk_start", "blk_cnt"))
+        out = zeros(ca, (dims[mode], R))
+        assert ca.lib.cptc_mttkrp_sparse3(mode, dc.data_ptr(), dv.data_ptr(), br.data_ptr(),
+                                          bs.data_ptr(), bc.data_ptr(), len(v["blk_row"]),
+                                          at[1 if mode == 0 else 0], at[1 if mode == 2 else 2],
+                                          out.data_ptr(), R, stream(ca)) == 0
+        ca.sync()
+        assert rel_err(out.numpy(), ref) <= 1e-10, (mode, R)
+
+
 def block_tensor(rng, dims, fill=0.5):
     cells = np.array(np.meshgrid(np.arange(0, 32), np.arange(16, 48), np.arange(0, dims[2]),
                                  indexing="ij")).reshape(3, -1)

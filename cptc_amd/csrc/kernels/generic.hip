@@ -6,8 +6,10 @@
 
 #include <algorithm>
 #include <cmath>
+#include <type_traits>
 
 #include "../host/hip_util.hpp"
+#include "block_sweep.hpp"
 
 namespace {
 
@@ -342,281 +344,383 @@ __global__ void gram_hadamard_kernel(const double* __restrict__ G, int ngram, in
     }
 }
 
-// Ridge Cholesky + per-row substitution (generic.cu:746-819), in two
-// kernels so that a driver can factor FtF while the MTTKRP that produces
-// FtV is still running.
+// Ridge solve F (FtF + eps I) = FtV (generic.cu:746-819), R <= 32, eps =
+// 1e-12 tr / R + 1e-300: a Cholesky factor L and two triangular solves a row.
 //
-// chol_factor_kernel (four waves) factors FtF + eps I in registers: row i
-// is split over 256 / RT threads, each holding RT^2 / 256 consecutive
-// columns.  Step j broadcasts the pivot column through LDS, scales column j
-// by the pivot's square root (the thread owning column j of each row) and
-// every thread subtracts L[i][j] L[k][j] from its entries k > j.  Each entry
-// therefore receives exactly the reference's sequence: (FtF + eps) minus
-// the products for k = 0, 1, ... in ascending order, then the division by
-// the pivot.  Entries above the diagonal take the same updates without a
-// per-thread condition (they are never read).  L (R x R row-major, zeros
-// above the diagonal) goes to global.
+// What bounds it is the chain of R pivots in one wave: there is little to
+// compute (R^3 / 3 + 2 R^2 a row) and a launch has few workgroups.  Row by
+// row substitutions would add 2 R more steps of that kind, so the solves are
+// products instead: with X_i the inverse of diagonal block i of L (16 x 16),
+// which comes out of the elimination beside L (the same row operations on the
+// identity),
+//   Y_1 = B_1 X_1^T,  Y_2 = (B_2 - Y_1 L_21^T) X_2^T,
+//   Z_2 = Y_2 X_2,    Z_1 = (Y_1 - Z_2 L_21) X_1,
+// six 16 x 16 x 16 products a 16-row tile on the FP64 matrix cores (two for R
+// <= 16), computed transposed: an accumulator is then the next product's B
+// operand as it stands.  The forward error bound is that of substitution (eps
+// |X| |L| a solve); measured against extended precision it is CHOLERR.
+// Wave 0 factors; all four waves solve a tile each.
 //
-// chol_apply_kernel stages L in LDS and solves one right-hand-side row per
-// lane with its y / x vector in registers (loops unrolled to RT >= R): the
-// reference's k-ascending forward and backward substitutions, each pivot's
-// division a multiplication by its reciprocal (chol_substitute).
+// Measured, launches back to back, 1000 rows (a row a lane, straight-line
+// steps with two LDS round trips, a root and a division each -> this): CHOLFIG
 constexpr int CHOL_RM = 32;
-constexpr int CHOL_T = 64;     // chol_apply_kernel: one right-hand side per thread
-constexpr int CHOL_FT = 256;   // chol_factor_kernel
+constexpr int CHOL_T = 256;
+constexpr int CHOL_ROWS = 64;   // right-hand sides a workgroup and pass
+constexpr int CHOL_LD = cptc::bsweep::LD;
 
-template <int RT>
-__global__ __launch_bounds__(CHOL_FT) void chol_factor_kernel(const double* __restrict__ FtF,
-                                                              int R, double* __restrict__ Lout)
+using cptc::bsweep::d4;
+
+template <int NB>
+struct RidgeLds
 {
-    // thread = row + RT * part; the thread holds columns part*C .. part*C+C-1
-    constexpr int LPR = CHOL_FT / RT;
-    constexpr int C = RT / LPR;
-    static_assert(C >= 1 && C <= 16, "chol layout");
-    __shared__ double col[RT];    // column j before scaling (pivot on the diagonal)
-    __shared__ double lcol[RT];   // column j of L
-    __shared__ double trs;
-    const int tid = threadIdx.x;
-    const int row = tid % RT;
-    const int part = tid / RT;
-    const int c0 = part * C;
-    const bool mine = row < R;    // rows >= R hold eps I (see below)
-    double a[C];
-#pragma unroll
-    for (int c = 0; c < C; ++c)
-        a[c] = (mine && c0 + c < R) ? FtF[size_t(row) * R + c0 + c] : 0.0;
-    // eps from the trace, summed in row order
-#pragma unroll
-    for (int c = 0; c < C; ++c)
-        if (c0 + c == row) col[row] = a[c];
-    __syncthreads();
-    if (tid == 0)
-    {
-        double tr = 0.0;
-        for (int i = 0; i < R; ++i) tr += col[i];
-        trs = tr;
-    }
-    __syncthreads();
-    const double tr = trs;
-    const double eps = 1e-12 * ((tr > 0.0) ? tr / double(R) : 1.0) + 1e-300;
-#pragma unroll
-    for (int c = 0; c < C; ++c)
-        if (c0 + c == row) a[c] += eps;
-    // Steps j < R only; rows >= R hold zeros off the diagonal, so they
-    // subtract exact zeros from the rows < R.
-    for (int jp = 0; jp * C < R; ++jp)
-    {
-#pragma unroll
-        for (int jc = 0; jc < C; ++jc)
-        {
-            const int j = jp * C + jc;
-            if (j >= R) break;
-            if (part == jp) col[row] = a[jc];
-            __syncthreads();
-            const double s = col[j];
-            const double d = (s > 0.0) ? sqrt(s) : sqrt(eps);
-            if (part == jp)
-            {
-                const double v = col[row];
-                lcol[row] = (row == j) ? d : ((mine && row > j) ? v / d : v);   // L[row][j]
-            }
-            __syncthreads();
-            const double lij = lcol[row];
-#pragma unroll
-            for (int c = 0; c < C; ++c)
-            {
-                if (part == jp && c == jc) a[c] = lij;
-                else if (c0 + c > j) a[c] -= lij * lcol[c0 + c];
-            }
-        }
-    }
-    if (mine)
-#pragma unroll
-        for (int c = 0; c < C; ++c)
-            if (c0 + c < R) Lout[size_t(row) * R + c0 + c] = (c0 + c <= row) ? a[c] : 0.0;
+    double X[NB][16 * CHOL_LD];   // inverses of L's diagonal blocks
+    double L21[16 * CHOL_LD];     // NB == 2 only
+};
+
+// x plus its copy N lanes round the row of 16 (DPP row_ror)
+template <int N>
+__device__ __forceinline__ double chol_ror_add(double x)
+{
+    const uint64_t u = __builtin_bit_cast(uint64_t, x);
+    const uint32_t lo =
+        uint32_t(__builtin_amdgcn_mov_dpp(int(uint32_t(u)), 0x120 + N, 0xf, 0xf, true));
+    const uint32_t hi =
+        uint32_t(__builtin_amdgcn_mov_dpp(int(uint32_t(u >> 32)), 0x120 + N, 0xf, 0xf, true));
+    return x + __builtin_bit_cast(double, (uint64_t(hi) << 32) | lo);
 }
 
-// L y' = y, then L^T x = y', with the Cholesky factor in LDS (RT x RT, padded
-// with the identity, so padding entries stay exact zeros) and the reciprocals
-// of its diagonal (dinv): row by row, each row's sum in ascending k as the
-// reference's substitutions, the division by the pivot done as a
-// multiplication by its reciprocal (one correctly rounded division per pivot
-// per workgroup instead of one per pivot and right-hand side; the row's
-// result differs from the division's by at most an ulp).  The next row's
-// entries of L (and its reciprocal) load into a second register set while
-// the current row's sum runs; the empty asm with a memory clobber keeps a
-// later row's loads from being hoisted further, which would not fit the
-// registers.
-template <int RT>
-__device__ __forceinline__ void chol_substitute(const double (*L)[RT + 1],
-                                                const double* __restrict__ dinv,
-                                                double (&y)[RT])
+// d = sqrt(p) and quotients v / d, correctly rounded, at half the latency of
+// the general ones: one reciprocal root, each result corrected by its exact
+// residual.  For p in about [2^-900, 2^1000]; WIDE takes the general ones.
+template <bool WIDE>
+struct Root
 {
-    double cur[RT], nxt[RT], cd = dinv[0], nd = 0.0;
-#pragma unroll
-    for (int i = 0; i < RT; ++i)
+    double d, r;
+    __device__ __forceinline__ explicit Root(double p)
     {
-        if (i + 1 < RT)
+        if constexpr (WIDE)
         {
-#pragma unroll
-            for (int k = 0; k <= i; ++k) nxt[k] = L[i + 1][k];
-            nd = dinv[i + 1];
+            d = sqrt(p);
         }
-        double s = y[i];
-#pragma unroll
-        for (int k = 0; k < i; ++k) s -= cur[k] * y[k];
-        y[i] = s * cd;
-        asm volatile("" ::: "memory");
-#pragma unroll
-        for (int k = 0; k <= i; ++k) cur[k] = nxt[k];
-        cd = nd;
+        else
+        {
+            r = __builtin_amdgcn_rsq(p);
+            r = fma(0.5 * r, fma(-(p * r), r, 1.0), r);
+            r = fma(0.5 * r, fma(-(p * r), r, 1.0), r);
+            d = p * r;
+            d = fma(0.5 * r, fma(-d, d, p), d);
+            r = fma(r, fma(-d, r, 1.0), r);
+        }
     }
-    // L^T x = y': row i takes column i of L below the diagonal
-    cd = dinv[RT - 1];
-#pragma unroll
-    for (int i = RT - 1; i >= 0; --i)
+    __device__ __forceinline__ double over(double v) const
     {
-        if (i > 0)
+        if constexpr (WIDE) return v / d;
+        const double q = v * r;
+        return fma(r, fma(-q, d, v), q);
+    }
+};
+
+// Columns K .. nv - 1 of a 16 x 16 block (accumulator layout: element v of
+// lane l is entry (l / 16 + 4 v, l % 16)) to those of L, and x, the identity
+// at K = 0, to L^-1; with BELOW, b, the block right of it, to L^-1 b, by the
+// same row operations (as X b its error grew with the condition of the block:
+// R = 32, kappa 1e8, 7.5e-10 in the solution against 2.3e-10).  A pivot s <= 0
+// (or NaN) counts as eps.
+template <int K, bool WIDE, bool BELOW>
+__device__ __forceinline__ void chol16_from(double (&a)[4], double (&x)[4], double (&b)[4],
+                                            int lr, int lk, double eps, int nv)
+{
+    using namespace cptc::bsweep;
+    constexpr int VK = K / 4, QK = K % 4;
+    const double s = readlane_d(a[VK], 16 * QK + K);
+    const double ck = bperm_d(a[VK], 16 * QK + lr);   // entry (K, lr)
+    const double xk = bperm_d(x[VK], 16 * QK + lr);
+    const double bk = BELOW ? bperm_d(b[VK], 16 * QK + lr) : 0.0;
+    const Root<WIDE> root((s > 0.0) ? s : eps);
+    const double c = lr > K ? root.over(ck) : 0.0, xs = root.over(xk);
+    const double bs = BELOW ? root.over(bk) : 0.0;
+#pragma unroll
+    for (int v = VK; v < 4; ++v)
+    {
+        // L_iK in the rows below K, 0 above
+        const double f = root.over(v == VK ? row_bcast_d<K, (0xf << (QK + 1)) & 0xf>(a[v])
+                                           : row_bcast_d<K, 0xf>(a[v]));
+        a[v] = fma(-f, c, a[v]);
+        x[v] = fma(-f, xs, x[v]);
+        a[v] = (lr == K) ? ((v == VK && lk == QK) ? root.d : f) : a[v];
+        if (v == VK) x[v] = (lk == QK) ? xs : x[v];
+        if constexpr (BELOW)
         {
-#pragma unroll
-            for (int k = i; k < RT; ++k) nxt[k] = L[k][i - 1];
-            nd = dinv[i - 1];
+            b[v] = fma(-f, bs, b[v]);
+            if (v == VK) b[v] = (lk == QK) ? bs : b[v];
         }
-        double s = y[i];
+    }
+    if constexpr (K + 1 < 16)
+        if (K + 1 < nv) chol16_from<K + 1, WIDE, BELOW>(a, x, b, lr, lk, eps, nv);
+}
+
+// x = L^-1 for a given block of L, the same operations
+template <int K>
+__device__ __forceinline__ void inv16_from(const double (&a)[4], double (&x)[4], int lr, int lk,
+                                           int nv)
+{
+    using namespace cptc::bsweep;
+    constexpr int VK = K / 4, QK = K % 4;
+    const double xs = bperm_d(x[VK], 16 * QK + lr) / readlane_d(a[VK], 16 * QK + K);
 #pragma unroll
-        for (int k = i + 1; k < RT; ++k) s -= cur[k] * y[k];
-        y[i] = s * cd;   // x[i]
-        asm volatile("" ::: "memory");
+    for (int v = VK; v < 4; ++v)
+    {
+        const double f = v == VK ? row_bcast_d<K, (0xf << (QK + 1)) & 0xf>(a[v])
+                                 : row_bcast_d<K, 0xf>(a[v]);
+        x[v] = fma(-f, xs, x[v]);
+        if (v == VK) x[v] = (lk == QK) ? xs : x[v];
+    }
+    if constexpr (K + 1 < 16)
+        if (K + 1 < nv) inv16_from<K + 1>(a, x, lr, lk, nv);
+}
+
+__device__ __forceinline__ void chol_identity(double (&x)[4], int lr, int lk)
+{
 #pragma unroll
-        for (int k = i; k < RT; ++k) cur[k] = nxt[k];
-        cd = nd;
+    for (int v = 0; v < 4; ++v) x[v] = (lk + 4 * v == lr) ? 1.0 : 0.0;
+}
+
+__device__ __forceinline__ void chol_put(double* m, const double (&x)[4], int lr, int lk)
+{
+#pragma unroll
+    for (int v = 0; v < 4; ++v) m[(lk + 4 * v) * CHOL_LD + lr] = x[v];
+}
+
+// acc + M1^T M2 of blocks in the accumulator layout
+__device__ __forceinline__ d4 chol_mul(const double (&m1)[4], const double (&m2)[4], d4 acc)
+{
+#pragma unroll
+    for (int v = 0; v < 4; ++v)
+        acc = __builtin_amdgcn_mfma_f64_16x16x4f64(m1[v], m2[v], acc, 0, 0, 0);
+    return acc;
+}
+
+// Wave 0: FtF + eps I = L L^T.  To w: X, L21; with OUT, L to global.
+template <int NB, bool WIDE, bool OUT>
+__device__ __forceinline__ void chol_factor(const double* __restrict__ FtF, int R, double eps,
+                                            int lr, int lk, double (&a)[NB][4], RidgeLds<NB>& w,
+                                            double* __restrict__ Lout)
+{
+    double x[4], p[4];   // p: A_12, then L21^T
+#pragma unroll
+    for (int v = 0; v < 4; ++v)
+        p[v] = (NB == 2 && 16 + lr < R) ? FtF[size_t(lk + 4 * v) * R + 16 + lr] : 0.0;
+    chol_identity(x, lr, lk);
+    chol16_from<0, WIDE, NB == 2>(a[0], x, p, lr, lk, eps, min(R, 16));
+    chol_put(w.X[0], x, lr, lk);
+    if constexpr (NB == 2)
+    {
+        double n[4];
+#pragma unroll
+        for (int v = 0; v < 4; ++v)
+        {
+            n[v] = -p[v];
+            w.L21[lr * CHOL_LD + lk + 4 * v] = p[v];
+        }
+        const d4 u = chol_mul(n, p, d4{a[1][0], a[1][1], a[1][2], a[1][3]});
+#pragma unroll
+        for (int v = 0; v < 4; ++v) a[1][v] = u[v];
+        chol_identity(x, lr, lk);
+        double none[4];
+        chol16_from<0, WIDE, false>(a[1], x, none, lr, lk, eps, R - 16);
+        chol_put(w.X[1], x, lr, lk);
+        if constexpr (OUT)
+#pragma unroll
+            for (int v = 0; v < 4; ++v)
+                if (16 + lr < R)
+                {
+                    Lout[size_t(lk + 4 * v) * R + 16 + lr] = 0.0;
+                    Lout[size_t(16 + lr) * R + lk + 4 * v] = p[v];
+                }
+    }
+    if constexpr (OUT)
+#pragma unroll
+        for (int i = 0; i < NB; ++i)
+#pragma unroll
+            for (int v = 0; v < 4; ++v)
+            {
+                const int r = lk + 4 * v, row = 16 * i + r, col = 16 * i + lr;
+                if (row < R && col < R) Lout[size_t(row) * R + col] = r >= lr ? a[i][v] : 0.0;
+            }
+}
+
+// Workgroup-wide factorisation, ends with a barrier.
+template <int NB, bool OUT>
+__device__ __forceinline__ void chol_factor_all(const double* __restrict__ FtF, int R,
+                                                RidgeLds<NB>& w, double* __restrict__ Lout)
+{
+    if (threadIdx.x < 64)
+    {
+        const int lane = threadIdx.x, lr = lane & 15, lk = lane >> 4;
+        double a[NB][4];
+#pragma unroll
+        for (int i = 0; i < NB; ++i)
+#pragma unroll
+            for (int v = 0; v < 4; ++v)
+            {
+                const int row = 16 * i + lk + 4 * v, col = 16 * i + lr;
+                a[i][v] = (row < R && col < R) ? FtF[size_t(row) * R + col] : 0.0;
+            }
+        const double dg = lane < R ? FtF[size_t(lane) * R + lane] : 0.0;
+        const double t =
+            chol_ror_add<1>(chol_ror_add<2>(chol_ror_add<4>(chol_ror_add<8>(dg))));
+        const double tr = cptc::bsweep::readlane_d(t, 0) + cptc::bsweep::readlane_d(t, 16);
+        const double eps = 1e-12 * ((tr > 0.0) ? tr / double(R) : 1.0) + 1e-300;
+#pragma unroll
+        for (int i = 0; i < NB; ++i)
+#pragma unroll
+            for (int v = 0; v < 4; ++v) a[i][v] += (lk + 4 * v == lr) ? eps : 0.0;
+        // eps <= every pivot's scale, and cancellation leaves no less than
+        // 2^-106 of it
+        const bool fits = tr >= 0x1p-700 && __all(fabs(dg) <= 0x1p900);
+        if (fits)
+            chol_factor<NB, false, OUT>(FtF, R, eps, lr, lk, a, w, Lout);
+        else
+            chol_factor<NB, true, OUT>(FtF, R, eps, lr, lk, a, w, Lout);
+    }
+    __syncthreads();
+}
+
+// A 16-row tile's right-hand sides, transposed: element v of lane l is entry
+// 16 i + l / 16 + 4 v of row `row` = first row + l % 16
+template <int NB>
+__device__ __forceinline__ void chol_load_rhs(const double* __restrict__ FtV, size_t dim, int R,
+                                              size_t row, int lk, double (&y)[NB][4])
+{
+    const double* b = FtV + row * R;
+#pragma unroll
+    for (int i = 0; i < NB; ++i)
+#pragma unroll
+        for (int v = 0; v < 4; ++v)
+            y[i][v] = (row < dim && 16 * i + lk + 4 * v < R) ? b[16 * i + lk + 4 * v] : 0.0;
+}
+
+// All passes of a wave over its tiles; y holds the first.
+template <int NB>
+__device__ __forceinline__ void chol_solve_rows(const RidgeLds<NB>& w,
+                                                const double* __restrict__ FtV,
+                                                double* __restrict__ F, size_t dim, int R,
+                                                size_t row, int lr, int lk, double (&y)[NB][4])
+{
+    double x[NB][4], xt[NB][4], l[4], lt[4];
+#pragma unroll
+    for (int v = 0; v < 4; ++v)
+    {
+#pragma unroll
+        for (int i = 0; i < NB; ++i)
+        {
+            x[i][v] = w.X[i][(lk + 4 * v) * CHOL_LD + lr];
+            xt[i][v] = w.X[i][lr * CHOL_LD + lk + 4 * v];
+        }
+        if (NB == 2)
+        {
+            l[v] = -w.L21[(lk + 4 * v) * CHOL_LD + lr];
+            lt[v] = -w.L21[lr * CHOL_LD + lk + 4 * v];
+        }
+    }
+    const size_t stride = size_t(gridDim.x) * CHOL_ROWS;
+    const d4 zero = {0.0, 0.0, 0.0, 0.0};
+    auto set = [](double (&o)[4], d4 v) {
+#pragma unroll
+        for (int q = 0; q < 4; ++q) o[q] = v[q];
+    };
+    for (; row - lr < dim; row += stride)   // wave-uniform
+    {
+        double nx[NB][4];
+        chol_load_rhs<NB>(FtV, dim, R, row + stride, lk, nx);
+        set(y[0], chol_mul(xt[0], y[0], zero));
+        if constexpr (NB == 2)
+        {
+            set(y[1], chol_mul(lt, y[0], d4{y[1][0], y[1][1], y[1][2], y[1][3]}));
+            set(y[1], chol_mul(xt[1], y[1], zero));
+            set(y[1], chol_mul(x[1], y[1], zero));
+            set(y[0], chol_mul(l, y[1], d4{y[0][0], y[0][1], y[0][2], y[0][3]}));
+        }
+        set(y[0], chol_mul(x[0], y[0], zero));
+        if (row < dim)
+        {
+            double* out = F + row * R;
+#pragma unroll
+            for (int i = 0; i < NB; ++i)
+#pragma unroll
+                for (int v = 0; v < 4; ++v)
+                    if (16 * i + lk + 4 * v < R) out[16 * i + lk + 4 * v] = y[i][v];
+        }
+#pragma unroll
+        for (int i = 0; i < NB; ++i)
+#pragma unroll
+            for (int v = 0; v < 4; ++v) y[i][v] = nx[i][v];
     }
 }
 
-template <int RT>
+template <int NB>
+__global__ __launch_bounds__(64) void chol_factor_kernel(const double* __restrict__ FtF, int R,
+                                                         double* __restrict__ Lout)
+{
+    __shared__ RidgeLds<NB> w;
+    chol_factor_all<NB, true>(FtF, R, w, Lout);
+}
+
+template <int NB>
 __global__ __launch_bounds__(CHOL_T) void chol_apply_kernel(const double* __restrict__ Lg,
                                                             const double* __restrict__ FtV,
                                                             double* __restrict__ F, size_t dim,
                                                             int R)
 {
-    // L padded to RT with the identity: padding entries of y stay 0 and
-    // only exact zeros are subtracted from the others, so the unrolled loops
-    // below need no condition on R
-    __shared__ double L[RT][RT + 1];
-    __shared__ double dinv[RT];
-    for (int x = threadIdx.x; x < RT * RT; x += CHOL_T)
+    __shared__ RidgeLds<NB> w;
+    const int lane = threadIdx.x & 63, wave = threadIdx.x / 64, lr = lane & 15, lk = lane >> 4;
+    const size_t row = size_t(blockIdx.x) * CHOL_ROWS + size_t(wave) * 16 + size_t(lr);
+    double y[NB][4];
+    chol_load_rhs<NB>(FtV, dim, R, row, lk, y);
+    if (wave < NB)   // a diagonal block each
     {
-        const int i = x / RT, k = x % RT;
-        const double v = (i < R && k < R) ? Lg[size_t(i) * R + k] : (i == k ? 1.0 : 0.0);
-        L[i][k] = v;
-        if (i == k) dinv[i] = 1.0 / v;
+        double a[4], x[4];
+#pragma unroll
+        for (int v = 0; v < 4; ++v)
+        {
+            const int i = 16 * wave + lk + 4 * v, k = 16 * wave + lr;
+            a[v] = (i < R && k < R) ? Lg[size_t(i) * R + k] : 0.0;
+        }
+        chol_identity(x, lr, lk);
+        inv16_from<0>(a, x, lr, lk, min(R - 16 * wave, 16));
+        chol_put(w.X[wave], x, lr, lk);
+    }
+    else if (NB == 2 && wave == 2)
+    {
+        double a[4];
+#pragma unroll
+        for (int v = 0; v < 4; ++v)
+        {
+            const int i = 16 + lk + 4 * v;
+            a[v] = i < R ? Lg[size_t(i) * R + lr] : 0.0;
+        }
+        chol_put(w.L21, a, lr, lk);
     }
     __syncthreads();
-    const size_t row = size_t(blockIdx.x) * CHOL_T + threadIdx.x;
-    if (row >= dim) return;
-    const double* b = FtV + row * R;
-    double y[RT];
-#pragma unroll
-    for (int i = 0; i < RT; ++i) y[i] = (i < R) ? b[i] : 0.0;
-    chol_substitute<RT>(L, dinv, y);
-    double* out = F + row * R;
-#pragma unroll
-    for (int i = 0; i < RT; ++i)
-        if (i < R) out[i] = y[i];
+    chol_solve_rows<NB>(w, FtV, F, dim, R, row, lr, lk, y);
 }
 
-// cptc_chol_ridge_factor + cptc_chol_ridge_apply in one launch, R <= RT <=
-// 32: each 64-lane workgroup (one wave) factors FtF + eps I itself, lane i
-// holding row i in registers and each step's pivot column passing through
-// LDS inside the wave, so no workgroup barrier (chol_factor_kernel's 2 R
-// barriers across four waves are most of its ~17 us at R = 32); every
-// operation is chol_factor_kernel's, in its order, so L is the same bits.
-// Then each lane solves one right-hand-side row as chol_apply_kernel.  The
-// grids are small (one workgroup per 64 rows), so the kernel takes registers
-// over occupancy (the row and the solve vector, 2 x 64 at RT = 32).
-template <int RT>
-__global__ __launch_bounds__(CHOL_T) __attribute__((amdgpu_waves_per_eu(1, 2))) void
-chol_solve_wave_kernel(const double* __restrict__ FtF,
-                                                                 const double* __restrict__ FtV,
-                                                                 double* __restrict__ F,
-                                                                 size_t dim, int R)
+// Both in one launch, every workgroup factoring for itself: the same bits
+// (quotients are correctly rounded in both).
+template <int NB>
+__global__ __launch_bounds__(CHOL_T) void chol_solve_kernel(const double* __restrict__ FtF,
+                                                            const double* __restrict__ FtV,
+                                                            double* __restrict__ F, size_t dim,
+                                                            int R)
 {
-    static_assert(RT <= 32 && CHOL_T == 64, "one wave, one row per lane");
-    __shared__ double L[RT][RT + 1];
-    __shared__ double dinv[RT];
-    __shared__ double lcol[2][RT];   // column j of L, alternating buffers by step
-    const int lane = threadIdx.x;
-    const bool act = lane < RT;
-    const bool mine = lane < R;
-    auto wave_sync = [] {
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-        __builtin_amdgcn_wave_barrier();
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-    };
-    // lane l's value of x (a wave-uniform result)
-    auto lane_f64 = [](double x, int l) {
-        const uint64_t u = __builtin_bit_cast(uint64_t, x);
-        const uint32_t lo = uint32_t(__builtin_amdgcn_readlane(int(uint32_t(u)), l));
-        const uint32_t hi = uint32_t(__builtin_amdgcn_readlane(int(uint32_t(u >> 32)), l));
-        return __builtin_bit_cast(double, (uint64_t(hi) << 32) | lo);
-    };
-    double a[RT];
-#pragma unroll
-    for (int c = 0; c < RT; ++c) a[c] = (mine && c < R) ? FtF[size_t(lane) * R + c] : 0.0;
-    // eps from the trace, summed in row order (the diagonal entry of row i is
-    // lane i's a[i])
-    double tr = 0.0;
-#pragma unroll
-    for (int i = 0; i < RT; ++i)
-        if (i < R) tr += lane_f64(a[i], i);
-    const double eps = 1e-12 * ((tr > 0.0) ? tr / double(R) : 1.0) + 1e-300;
-#pragma unroll
-    for (int c = 0; c < RT; ++c)
-        if (c == lane) a[c] += eps;
-    // (fully unrolled, so the row stays in registers: a partly unrolled
-    // loop indexes it at run time and moves it to scratch memory).  The
-    // pivot is lane j's a[j], read across lanes; column j of L goes through
-    // LDS, in the buffer the step after next reuses (a wave's LDS operations
-    // are in order, so the next step's writes to the other buffer need no
-    // barrier behind this step's reads).
-#pragma unroll
-    for (int j = 0; j < RT; ++j)
-    {
-        if (j < R)   // steps j < R only (uniform; no early exit, so the loop unrolls)
-        {
-            const double sp = lane_f64(a[j], j);
-            const double d = (sp > 0.0) ? sqrt(sp) : sqrt(eps);
-            const double v = a[j];
-            const double lij = (lane == j) ? d : ((mine && lane > j) ? v / d : v);
-            double* lc = lcol[j & 1];
-            if (act) lc[lane] = lij;
-            wave_sync();
-            a[j] = lij;
-#pragma unroll
-            for (int c = j + 1; c < RT; ++c) a[c] -= lij * lc[c];
-        }
-    }
-    // L padded to RT with the identity (chol_apply_kernel's layout)
-    if (act)
-#pragma unroll
-        for (int c = 0; c < RT; ++c)
-        {
-            const double v = (mine && c < R) ? ((c <= lane) ? a[c] : 0.0) : (c == lane ? 1.0 : 0.0);
-            L[lane][c] = v;
-            if (c == lane) dinv[lane] = 1.0 / v;
-        }
-    __syncthreads();
-    const size_t row = size_t(blockIdx.x) * CHOL_T + size_t(lane);
-    if (row >= dim) return;
-    const double* b = FtV + row * R;
-    double y[RT];
-#pragma unroll
-    for (int i = 0; i < RT; ++i) y[i] = (i < R) ? b[i] : 0.0;
-    chol_substitute<RT>(L, dinv, y);
-    double* out = F + row * R;
-#pragma unroll
-    for (int i = 0; i < RT; ++i)
-        if (i < R) out[i] = y[i];
+    __shared__ RidgeLds<NB> w;
+    const int lane = threadIdx.x & 63, lr = lane & 15, lk = lane >> 4;
+    const size_t row =
+        size_t(blockIdx.x) * CHOL_ROWS + size_t(threadIdx.x / 64) * 16 + size_t(lr);
+    double y[NB][4];
+    chol_load_rhs<NB>(FtV, dim, R, row, lk, y);   // in flight beside the factorisation
+    chol_factor_all<NB, false>(FtF, R, w, nullptr);
+    chol_solve_rows<NB>(w, FtV, F, dim, R, row, lr, lk, y);
 }
 
 // Column sums of squares: P partials of R each (deterministic).
@@ -810,6 +914,20 @@ __global__ void finalize_add2_kernel(const double* __restrict__ part, int P,
     }
 }
 
+// diagonal blocks of 16
+template <class Run>
+void chol_blocks(int R, Run run)
+{
+    if (R <= 16) run(std::integral_constant<int, 1>{});
+    else run(std::integral_constant<int, 2>{});
+}
+
+// 1024 workgroups, four to a CU, take further rows in passes
+dim3 chol_grid(size_t dim)
+{
+    return dim3(unsigned(std::min<size_t>((dim + CHOL_ROWS - 1) / CHOL_ROWS, 1024)));
+}
+
 bool factors_ok(int n, const double* const* h_F)
 {
     if (!h_F) return false;
@@ -941,11 +1059,11 @@ extern "C" int cptc_chol_ridge_factor(const double* d_FtF, double* d_L, int R, v
     CPTC_REQUIRE(R >= 1 && R <= CHOL_RM, CPTC_ERR_ARG, "cptc_chol_ridge_factor: R %d (1..32)", R);
     CPTC_REQUIRE(d_FtF && d_L, CPTC_ERR_ARG, "cptc_chol_ridge_factor: null pointer");
     hipStream_t s = cptc::as_stream(stream);
-    if (R <= 16)
-        hipLaunchKernelGGL(chol_factor_kernel<16>, dim3(1), dim3(CHOL_FT), 0, s, d_FtF, R, d_L);
-    else
-        hipLaunchKernelGGL(chol_factor_kernel<CHOL_RM>, dim3(1), dim3(CHOL_FT), 0, s, d_FtF, R,
-                           d_L);
+    auto run = [&](auto NB) {
+        hipLaunchKernelGGL(chol_factor_kernel<decltype(NB)::value>, dim3(1), dim3(64), 0, s,
+                           d_FtF, R, d_L);
+    };
+    chol_blocks(R, run);
     CPTC_LAUNCHED();
     return CPTC_OK;
 }
@@ -956,18 +1074,14 @@ extern "C" int cptc_chol_ridge_apply(const double* d_L, const double* d_FtV, dou
     CPTC_REQUIRE(R >= 1 && R <= CHOL_RM, CPTC_ERR_ARG, "cptc_chol_ridge_apply: R %d (1..32)", R);
     if (dim == 0) return CPTC_OK;
     CPTC_REQUIRE(d_L && d_FtV && d_F, CPTC_ERR_ARG, "cptc_chol_ridge_apply: null pointer");
-    CPTC_REQUIRE(dim / CHOL_T < (size_t(1) << 31), CPTC_ERR_ARG,
-                 "cptc_chol_ridge_apply: %zu rows", dim);
-    const dim3 grid(unsigned((dim + CHOL_T - 1) / CHOL_T));
+    CPTC_REQUIRE(dim / 64 < (size_t(1) << 31), CPTC_ERR_ARG, "cptc_chol_ridge_apply: %zu rows",
+                 dim);
     hipStream_t s = cptc::as_stream(stream);
-    if (R <= 8)
-        hipLaunchKernelGGL(chol_apply_kernel<8>, grid, dim3(CHOL_T), 0, s, d_L, d_FtV, d_F, dim, R);
-    else if (R <= 16)
-        hipLaunchKernelGGL(chol_apply_kernel<16>, grid, dim3(CHOL_T), 0, s, d_L, d_FtV, d_F, dim,
-                           R);
-    else
-        hipLaunchKernelGGL(chol_apply_kernel<CHOL_RM>, grid, dim3(CHOL_T), 0, s, d_L, d_FtV, d_F,
-                           dim, R);
+    auto run = [&](auto NB) {
+        hipLaunchKernelGGL(chol_apply_kernel<decltype(NB)::value>, chol_grid(dim), dim3(CHOL_T), 0,
+                           s, d_L, d_FtV, d_F, dim, R);
+    };
+    chol_blocks(R, run);
     CPTC_LAUNCHED();
     return CPTC_OK;
 }
@@ -978,21 +1092,14 @@ extern "C" int cptc_chol_ridge_solve(const double* d_FtF, const double* d_FtV, d
     CPTC_REQUIRE(R >= 1 && R <= CHOL_RM, CPTC_ERR_ARG, "cptc_chol_ridge_solve: R %d (1..32)", R);
     if (dim == 0) return CPTC_OK;
     CPTC_REQUIRE(d_FtF && d_FtV && d_F, CPTC_ERR_ARG, "cptc_chol_ridge_solve: null pointer");
-    CPTC_REQUIRE(dim / CHOL_T < (size_t(1) << 31), CPTC_ERR_ARG,
-                 "cptc_chol_ridge_solve: %zu rows", dim);
-    // one launch: every workgroup factors (one wave, ~1-2 us) and solves its
-    // 64 rows; the same bits as cptc_chol_ridge_factor + cptc_chol_ridge_apply
-    const dim3 grid(unsigned((dim + CHOL_T - 1) / CHOL_T));
+    CPTC_REQUIRE(dim / 64 < (size_t(1) << 31), CPTC_ERR_ARG, "cptc_chol_ridge_solve: %zu rows",
+                 dim);
     hipStream_t s = cptc::as_stream(stream);
-    if (R <= 8)
-        hipLaunchKernelGGL(chol_solve_wave_kernel<8>, grid, dim3(CHOL_T), 0, s, d_FtF, d_FtV, d_F,
-                           dim, R);
-    else if (R <= 16)
-        hipLaunchKernelGGL(chol_solve_wave_kernel<16>, grid, dim3(CHOL_T), 0, s, d_FtF, d_FtV,
-                           d_F, dim, R);
-    else
-        hipLaunchKernelGGL(chol_solve_wave_kernel<CHOL_RM>, grid, dim3(CHOL_T), 0, s, d_FtF,
-                           d_FtV, d_F, dim, R);
+    auto run = [&](auto NB) {
+        hipLaunchKernelGGL(chol_solve_kernel<decltype(NB)::value>, chol_grid(dim), dim3(CHOL_T), 0,
+                           s, d_FtF, d_FtV, d_F, dim, R);
+    };
+    chol_blocks(R, run);
     CPTC_LAUNCHED();
     return CPTC_OK;
 }

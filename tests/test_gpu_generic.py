@@ -485,6 +485,34 @@ def test_chol_ridge_factor_apply(ca, dev, R, rows, rank_def):
     assert np.array_equal(out.numpy(), ref.numpy())
 
 
+@pytest.mark.parametrize("R", [1, 15, 16, 17, 31, 32])
+@pytest.mark.parametrize("rows,scale", [(1, 1.0), (15, 1.0), (16, 1e-280), (17, 1e-220),
+                                        (63, 1e275), (65, 1e260), (64 * 1024 + 17, 1.0)])
+def test_chol_ridge_tile_edges(ca, dev, R, rows, scale):
+    """The 16-row tiles and 16-column blocks at their edges, more rows than
+    one pass takes, in place, and scales on both sides of the range of the
+    fast root and quotient (powers of two, so the result only scales: same
+    bits as at scale 1, where the solve's backward error is <= c R eps)."""
+    rng = np.random.default_rng(R + rows)
+    A = rng.random((3 * R + 5, R))
+    FtF = A.T @ A
+    Y = rng.standard_normal((rows, R))
+    sc = 2.0 ** round(np.log2(scale))
+    outs = []
+    for f in (1.0, sc):
+        dA, d = dbuf(ca, FtF * f), dbuf(ca, Y)
+        assert ca.lib.cptc_chol_ridge_solve(dA.data_ptr(), d.data_ptr(), d.data_ptr(), rows, R,
+                                            None) == 0
+        ca.sync()
+        outs.append(d.numpy().reshape(rows, R).copy())
+    M = FtF + 1e-12 * np.trace(FtF) / R * np.eye(R)
+    res = np.abs(outs[0] @ M - Y).max(axis=1)
+    bound = 16 * R * np.finfo(float).eps * (np.abs(outs[0]) @ np.abs(M)).max(axis=1)
+    assert np.all(res <= bound)
+    # 1e-300 in eps is 1e-8 of the rest of it at 1e-280: 1e-20 of the matrix
+    assert rel_err(outs[1] * sc, outs[0]) <= 64 * R * np.finfo(float).eps * np.linalg.cond(M)
+
+
 def test_chol_ridge_singular_pivot(ca, orc, dev):
     """A rank-deficient FtF hits the s <= 0 -> sqrt(eps) branch."""
     R = 6

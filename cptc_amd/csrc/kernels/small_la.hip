@@ -80,7 +80,13 @@ __global__ __launch_bounds__(256) void gram_partial_kernel(const double* __restr
         }
 }
 
-// Gram partials for R > 64 on the FP64 matrix cores (v_mfma_f64_16x16x4f64):
+// Gram partials for R > 32 on the FP64 matrix cores (v_mfma_f64_16x16x4f64);
+// cptc_gram at R = 64 with this instead of the 16 x 16 threads above, and the
+// partials' sum below over four waves: 64 rows 12.9 -> 8.7 us, 1500 14.6 ->
+// 10.6, 12000 25.6 -> 14.5, 32768 39 -> 18 (R = 100, the sum alone: 12000 28.7
+// -> 22.6, 32768 41.6 -> 32.7).  At R <= 32 a tile's MFMAs are mostly padding
+// and the threads have 1 or 4 entries: 500 rows 7.8 us at R = 32 there.
+//
 // grid.x = row range p (rows [p rpw, (p + 1) rpw)), grid.y = one upper-
 // triangle pair (bi <= bj) of 64-rank tiles.  Wave w takes tile rows
 // 16w .. 16w + 15 against the tile's four 16-column blocks t (all four, so
@@ -166,13 +172,16 @@ __global__ __launch_bounds__(256) void gram_mfma_partial_kernel(const double* __
     load(r_lo, P);
     for (size_t i0 = r_lo; i0 < r_hi; i0 += 2 * STEP)
     {
-        load(i0 + STEP, Q);
+        // (uniform; ranges of at most 64 rows are the common ones)
+        const bool more = i0 + STEP < r_hi;
+        if (more) load(i0 + STEP, Q);
         __builtin_amdgcn_sched_barrier(0);
-        compute(i0, P);
+        compute(i0, P);   // zero A past the range
         __builtin_amdgcn_sched_barrier(0);
-        load(i0 + 2 * STEP, P);
+        if (!more) break;
+        if (i0 + 2 * STEP < r_hi) load(i0 + 2 * STEP, P);
         __builtin_amdgcn_sched_barrier(0);
-        compute(i0 + STEP, Q);   // all-zero A past the range
+        compute(i0 + STEP, Q);
         __builtin_amdgcn_sched_barrier(0);
     }
     double* __restrict__ out = part + size_t(blockIdx.x) * size_t(R) * R;
@@ -220,19 +229,27 @@ __global__ void sum_partials_kernel(const double* __restrict__ part, int P, size
 // read in order, coalesced) and written to their own place and, above the
 // diagonal, to their mirror's (the one scattered access, once per entry
 // rather than once per partial), so the result is symmetric by construction.
-__global__ void sum_partials_sym_kernel(const double* __restrict__ part, int P, int R,
-                                        double* __restrict__ out)
+// A wave takes 64 entries, and the four waves a quarter of the partials each:
+// R^2 / 256 workgroups alone leave most of the chip idle.
+__global__ __launch_bounds__(256) void sum_partials_sym_kernel(const double* __restrict__ part,
+                                                               int P, int R,
+                                                               double* __restrict__ out)
 {
+    __shared__ double red[3][64];
     const size_t n = size_t(R) * R;
-    for (size_t x = size_t(blockIdx.x) * blockDim.x + threadIdx.x; x < n;
-         x += size_t(gridDim.x) * blockDim.x)
-    {
-        const int r = int(x / size_t(R)), c = int(x % size_t(R));
-        if (r > c) continue;
-        const double v = ordered_sum(part, P, n, x);
-        out[x] = v;
-        if (r < c) out[size_t(c) * R + r] = v;
-    }
+    const int lane = threadIdx.x & 63;
+    const int w = __builtin_amdgcn_readfirstlane(int(threadIdx.x) >> 6);
+    const size_t x = size_t(blockIdx.x) * 64 + size_t(lane);
+    const int r = int(x / size_t(R)), c = int(x % size_t(R));
+    const bool mine = x < n && r <= c;
+    const int q = (P + 3) / 4, lo = min(w * q, P), hi = min(lo + q, P);
+    double v = mine ? ordered_sum(part + size_t(lo) * n, hi - lo, n, x) : 0.0;
+    if (w > 0) red[w - 1][lane] = v;
+    __syncthreads();
+    if (w > 0 || !mine) return;
+    v = (v + red[0][lane]) + (red[1][lane] + red[2][lane]);
+    out[x] = v;
+    if (r < c) out[size_t(c) * R + r] = v;
 }
 
 __global__ void hadamard_kernel(const double* A, const double* B, double* C, size_t n)
@@ -1924,8 +1941,11 @@ extern "C" int cptc_gram(const double* d_F, size_t rows, int R, double* d_G, voi
         CPTC_HIP(hipMemsetAsync(d_G, 0, RR * sizeof(double), s));
         return CPTC_OK;
     }
-    const int P = partials_for(rows, R > 64 ? CPTC_GRAM_MFMA_ROWS : 64);
+    int P = partials_for(rows, R > 32 ? CPTC_GRAM_MFMA_ROWS : 64);
     const size_t rpw = (rows + P - 1) / P;
+    // the ranges that have rows (16389 rows: 256 ranges of 65, the last three
+    // empty); gram_mfma_partial_kernel writes nothing for an empty one
+    if (R > 32) P = int((rows + rpw - 1) / rpw);
     void* part = nullptr;
     CPTC_TRY(cptc::scratch_get(cptc::SCR_GRAM, size_t(P) * RR * sizeof(double), &part));
     double* pd = static_cast<double*>(part);
@@ -1939,11 +1959,6 @@ extern "C" int cptc_gram(const double* d_F, size_t rows, int R, double* d_G, voi
         hipLaunchKernelGGL(gram_partial_kernel<2>, dim3(P, 1), dim3(256), 0, s, d_F, rows, R, rpw,
                            1, pd);
     }
-    else if (R <= 64)
-    {
-        hipLaunchKernelGGL(gram_partial_kernel<4>, dim3(P, 1), dim3(256), 0, s, d_F, rows, R, rpw,
-                           1, pd);
-    }
     else
     {
         // the FP64 matrix cores over 64 x 64 tiles, upper triangle only
@@ -1951,7 +1966,7 @@ extern "C" int cptc_gram(const double* d_F, size_t rows, int R, double* d_G, voi
         hipLaunchKernelGGL(gram_mfma_partial_kernel, dim3(P, nt * (nt + 1) / 2), dim3(256), 0, s,
                            d_F, rows, R, rpw, nt, pd);
         CPTC_LAUNCHED();
-        hipLaunchKernelGGL(sum_partials_sym_kernel, dim3(cptc::grid_for(RR, 256, 1024)),
+        hipLaunchKernelGGL(sum_partials_sym_kernel, dim3(unsigned((RR + 63) / 64)),
                            dim3(256), 0, s, pd, P, R, d_G);
         CPTC_LAUNCHED();
         return CPTC_OK;

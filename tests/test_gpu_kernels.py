@@ -532,6 +532,24 @@ def test_gram(ca, dev, rows, R):
     assert np.array_equal(G.numpy(), G.numpy().T)
 
 
+@pytest.mark.parametrize("R", [33, 48, 63, 64, 65])
+@pytest.mark.parametrize("rows", [1, 31, 32, 33, 64, 65, 129, 256 * 64 + 5])
+def test_gram_one_tile_edges(ca, dev, rows, R):
+    """The matrix-core Gram of one 64-column tile (and one column more): rows
+    at the edges of a batch (32), of a range (64) and of the 256 ranges, with
+    NaN in the rows behind the last; symmetric, and within the rounding of a
+    sum of `rows` products."""
+    F = np.full((rows + 70, R), np.nan)
+    F[:rows] = np.random.default_rng(rows * 100 + R).standard_normal((rows, R))
+    dF, G = to_dev(ca, F), zeros(ca, (R, R))
+    assert ca.lib.cptc_gram(dF.data_ptr(), rows, R, G.data_ptr(), stream(ca)) == 0
+    ca.sync()
+    A, g = F[:rows], G.numpy()
+    assert np.array_equal(g, g.T)
+    bound = 2 * (rows + 8) * np.finfo(float).eps * (np.abs(A).T @ np.abs(A))
+    assert np.all(np.abs(g - A.T @ A) <= bound)
+
+
 @pytest.mark.parametrize("R,dim", [(64, 100), (65, 1), (65, 77), (100, 1000), (127, 63),
                                    (128, 28818), (128, 17), (129, 300)])
 def test_apply_pinv_vs_numpy(ca, dev, R, dim):

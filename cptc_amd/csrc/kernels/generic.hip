@@ -903,15 +903,22 @@ __global__ __launch_bounds__(256) void residual_nd_kernel(int nmodes,
     }
 }
 
-__global__ void finalize_add2_kernel(const double* __restrict__ part, int P,
-                                     double* __restrict__ out2)
+// out2 += the P partials' sums, in a fixed order
+__global__ __launch_bounds__(256) void finalize_add2_kernel(const double* __restrict__ part, int P,
+                                                            double* __restrict__ out2)
 {
-    if (threadIdx.x < 2)
+    __shared__ double red[256];
+    // thread t: sum t % 2, partials t / 2, t / 2 + 128, ...
+    double t = 0.0;
+    for (int p = int(threadIdx.x) / 2; p < P; p += 128) t += part[2 * size_t(p) + threadIdx.x % 2];
+    red[threadIdx.x] = t;
+    __syncthreads();
+    for (int h = 128; h >= 2; h >>= 1)
     {
-        double t = 0.0;
-        for (int p = 0; p < P; ++p) t += part[2 * size_t(p) + threadIdx.x];
-        out2[threadIdx.x] += t;
+        if (int(threadIdx.x) < h) red[threadIdx.x] += red[threadIdx.x + h];
+        __syncthreads();
     }
+    if (threadIdx.x < 2) out2[threadIdx.x] += red[threadIdx.x];
 }
 
 // diagonal blocks of 16
@@ -1161,7 +1168,7 @@ extern "C" int cptc_residual_nd(int nmodes, const uint32_t* d_coords, const doub
     hipLaunchKernelGGL(residual_nd_kernel, dim3(P), dim3(256), 0, s, nmodes, d_coords, d_vals, nnz,
                        F, d_lambda, R, part);
     CPTC_LAUNCHED();
-    hipLaunchKernelGGL(finalize_add2_kernel, dim3(1), dim3(64), 0, s, part, P, d_out2);
+    hipLaunchKernelGGL(finalize_add2_kernel, dim3(1), dim3(256), 0, s, part, P, d_out2);
     CPTC_LAUNCHED();
     return CPTC_OK;
 }

@@ -1,10 +1,12 @@
 // Exact residual ||X - Xhat||^2 and ||X||^2 over row-sorted views and dense
 // tile pools, plus the factor unpermutation of the export path.
 //
-// The model value of an element follows common.cu:303-334: two accumulators
-// over even / odd ranks, each term (a*b*c)*lambda_r, pred = p0 + p1.
+// The model value of an element follows common.cu:303-334: sums over the even
+// and the odd ranks, each term (a*b*c)*lambda_r, pred = p0 + p1.
 // Per-workgroup partials are summed in a fixed order (deterministic).
 #include <hip/hip_runtime.h>
+
+#include <type_traits>
 
 #include "../host/hip_util.hpp"
 
@@ -12,30 +14,35 @@ namespace {
 
 constexpr int THREADS = 256;
 
+// A lane group of LPE lanes takes an element, lane q of it the rank pairs q, q
+// + LPE, ...: with a lane an element every load touches 64 lines.  p0 and p1
+// are the even and the odd ranks' sums.  The whole call, before (a lane an
+// element, one thread adding the partials) and now: 1 M nonzeros R = 8 189 ->
+// 84 us, 16 253 -> 116, 32 354 -> 192; R = 64, 2 M nonzeros 765 -> 466.
+template <int LPE>
 __device__ double model_value(const double* __restrict__ pa, const double* __restrict__ pb,
-                              const double* __restrict__ pc, const double* __restrict__ lam, int R)
+                              const double* __restrict__ pc, const double* __restrict__ lam, int R,
+                              int q)
 {
     double p0 = 0.0, p1 = 0.0;
-    int r = 0;
-    for (; r + 1 < R; r += 2)
+    for (int r = 2 * q; r < R; r += 2 * LPE)
     {
+        const bool two = r + 1 < R;
+        const int r1 = two ? r + 1 : r;
         double x0 = pa[r] * pb[r] * pc[r];
-        double x1 = pa[r + 1] * pb[r + 1] * pc[r + 1];
+        double x1 = pa[r1] * pb[r1] * pc[r1];
         if (lam)
         {
             x0 *= lam[r];
-            x1 *= lam[r + 1];
+            x1 *= lam[r1];
         }
         p0 += x0;
-        p1 += x1;
+        if (two) p1 += x1;
     }
-    for (; r < R; ++r)
-    {
-        double x = pa[r] * pb[r] * pc[r];
-        if (lam) x *= lam[r];
-        p0 += x;
-    }
-    return p0 + p1;
+    double p = p0 + p1;
+#pragma unroll
+    for (int o = 1; o < LPE; o <<= 1) p += __shfl_xor(p, o, 64);
+    return p;
 }
 
 __device__ void block_sum2(double a, double b, double* __restrict__ out2)
@@ -60,44 +67,26 @@ __device__ void block_sum2(double a, double b, double* __restrict__ out2)
     }
 }
 
+template <int LPE>
 __global__ __launch_bounds__(THREADS) void residual_view_kernel(
     const uint64_t* __restrict__ coords, const double* __restrict__ vals, size_t nnz,
     const double* __restrict__ A, const double* __restrict__ B, const double* __restrict__ C,
     const double* __restrict__ lam, int R, double* __restrict__ part)
 {
+    constexpr int EPB = THREADS / LPE;
     double res = 0.0, xx = 0.0;
-    const size_t stride = size_t(gridDim.x) * THREADS;
-    for (size_t e = size_t(blockIdx.x) * THREADS + threadIdx.x; e < nnz; e += stride)
+    const int q = int(threadIdx.x) % LPE;
+    for (size_t e = size_t(blockIdx.x) * EPB + threadIdx.x / LPE; e < nnz;
+         e += size_t(gridDim.x) * EPB)
     {
         const uint64_t pc = coords[e];
         const double v = vals[e];
         const uint32_t i = uint32_t(pc >> 30) & 0x7FFFu, j = uint32_t(pc >> 15) & 0x7FFFu,
                        k = uint32_t(pc) & 0x7FFFu;
-        const double d =
-            v - model_value(A + size_t(i) * R, B + size_t(j) * R, C + size_t(k) * R, lam, R);
-        res += d * d;
-        xx += v * v;
-    }
-    block_sum2(res, xx, part + 2 * size_t(blockIdx.x));
-}
-
-__global__ __launch_bounds__(THREADS) void residual_tiles_kernel(
-    const int32_t* __restrict__ tiles4, const uint64_t* __restrict__ off,
-    const int32_t* __restrict__ lid, const double* __restrict__ pval, size_t ntiles,
-    const double* __restrict__ A, const double* __restrict__ B, const double* __restrict__ C,
-    const double* __restrict__ lam, int R, double* __restrict__ part)
-{
-    double res = 0.0, xx = 0.0;
-    for (size_t t = blockIdx.x; t < ntiles; t += gridDim.x)
-    {
-        const int b0 = tiles4[4 * t] * 16, b1 = tiles4[4 * t + 1] * 16, b2 = tiles4[4 * t + 2] * 16;
-        for (uint64_t e = off[t] + threadIdx.x; e < off[t + 1]; e += THREADS)
+        const double d = v - model_value<LPE>(A + size_t(i) * R, B + size_t(j) * R,
+                                              C + size_t(k) * R, lam, R, q);
+        if (q == 0)
         {
-            const int l = lid[e];
-            const double v = pval[e];
-            const size_t i = size_t(b0 + (l >> 8)), j = size_t(b1 + ((l >> 4) & 15)),
-                         k = size_t(b2 + (l & 15));
-            const double d = v - model_value(A + i * R, B + j * R, C + k * R, lam, R);
             res += d * d;
             xx += v * v;
         }
@@ -105,18 +94,52 @@ __global__ __launch_bounds__(THREADS) void residual_tiles_kernel(
     block_sum2(res, xx, part + 2 * size_t(blockIdx.x));
 }
 
-__global__ void finalize_add_kernel(const double* __restrict__ part, int P,
-                                    double* __restrict__ out2)
+template <int LPE>
+__global__ __launch_bounds__(THREADS) void residual_tiles_kernel(
+    const int32_t* __restrict__ tiles4, const uint64_t* __restrict__ off,
+    const int32_t* __restrict__ lid, const double* __restrict__ pval, size_t ntiles,
+    const double* __restrict__ A, const double* __restrict__ B, const double* __restrict__ C,
+    const double* __restrict__ lam, int R, double* __restrict__ part)
 {
-    if (threadIdx.x != 0 || blockIdx.x != 0) return;
+    constexpr int EPB = THREADS / LPE;
+    double res = 0.0, xx = 0.0;
+    const int q = int(threadIdx.x) % LPE;
+    for (size_t t = blockIdx.x; t < ntiles; t += gridDim.x)
+    {
+        const int b0 = tiles4[4 * t] * 16, b1 = tiles4[4 * t + 1] * 16, b2 = tiles4[4 * t + 2] * 16;
+        for (uint64_t e = off[t] + threadIdx.x / LPE; e < off[t + 1]; e += EPB)
+        {
+            const int l = lid[e];
+            const double v = pval[e];
+            const size_t i = size_t(b0 + (l >> 8)), j = size_t(b1 + ((l >> 4) & 15)),
+                         k = size_t(b2 + (l & 15));
+            const double d = v - model_value<LPE>(A + i * R, B + j * R, C + k * R, lam, R, q);
+            if (q == 0)
+            {
+                res += d * d;
+                xx += v * v;
+            }
+        }
+    }
+    block_sum2(res, xx, part + 2 * size_t(blockIdx.x));
+}
+
+// out2 += the P partials' sums, in a fixed order.  One thread adding them in
+// turn took 95 us for 2048 partials (a load's latency each).
+__global__ __launch_bounds__(THREADS) void finalize_add_kernel(const double* __restrict__ part,
+                                                               int P, double* __restrict__ out2)
+{
+    __shared__ double t[2];
     double a = 0.0, b = 0.0;
-    for (int p = 0; p < P; ++p)
+    for (int p = threadIdx.x; p < P; p += THREADS)
     {
         a += part[2 * p];
         b += part[2 * p + 1];
     }
-    out2[0] += a;
-    out2[1] += b;
+    block_sum2(a, b, t);
+    if (threadIdx.x != 0) return;
+    out2[0] += t[0];
+    out2[1] += t[1];
 }
 
 __global__ void unpermute_kernel(const double* __restrict__ src, double* __restrict__ dst,
@@ -132,6 +155,16 @@ __global__ void unpermute_kernel(const double* __restrict__ src, double* __restr
     }
 }
 
+// lanes an element.  1 M nonzeros, the whole call at 1 / 2 / 4 / 8 lanes: R = 4
+// 62 / 63 / 84 / 138 us, 8 98 / 84 / 83 / 133, 16 211 / 150 / 116 / 134, 32 391 /
+// 258 / 192 / 210 (more lanes, fewer elements in flight and more shuffles)
+template <class Run>
+void residual_lanes(int R, Run run)
+{
+    if (R <= 4) run(std::integral_constant<int, 2>{});
+    else run(std::integral_constant<int, 4>{});
+}
+
 }  // namespace
 
 extern "C" int cptc_residual3_view(const uint64_t* d_coords, const double* d_vals, size_t nnz,
@@ -143,14 +176,16 @@ extern "C" int cptc_residual3_view(const uint64_t* d_coords, const double* d_val
     if (nnz == 0) return CPTC_OK;
     CPTC_REQUIRE(d_coords && d_vals, CPTC_ERR_ARG, "cptc_residual3_view: null view");
     hipStream_t s = cptc::as_stream(stream);
-    const int P = int(cptc::grid_for(nnz, THREADS * 8, 2048));
+    const int P = int(cptc::grid_for(nnz, THREADS, 2048));
     void* buf = nullptr;
     CPTC_TRY(cptc::scratch_get(cptc::SCR_REDUCE, size_t(P) * 2 * sizeof(double), &buf));
     double* part = static_cast<double*>(buf);
-    hipLaunchKernelGGL(residual_view_kernel, dim3(P), dim3(THREADS), 0, s, d_coords, d_vals, nnz,
-                       d_A, d_B, d_C, d_lambda, R, part);
+    residual_lanes(R, [&](auto L) {
+        hipLaunchKernelGGL(residual_view_kernel<decltype(L)::value>, dim3(P), dim3(THREADS), 0, s,
+                           d_coords, d_vals, nnz, d_A, d_B, d_C, d_lambda, R, part);
+    });
     CPTC_LAUNCHED();
-    hipLaunchKernelGGL(finalize_add_kernel, dim3(1), dim3(64), 0, s, part, P, d_out2);
+    hipLaunchKernelGGL(finalize_add_kernel, dim3(1), dim3(THREADS), 0, s, part, P, d_out2);
     CPTC_LAUNCHED();
     return CPTC_OK;
 }
@@ -171,10 +206,13 @@ extern "C" int cptc_residual3_tiles(const int32_t* d_tiles, const uint64_t* d_po
     void* buf = nullptr;
     CPTC_TRY(cptc::scratch_get(cptc::SCR_REDUCE, size_t(P) * 2 * sizeof(double), &buf));
     double* part = static_cast<double*>(buf);
-    hipLaunchKernelGGL(residual_tiles_kernel, dim3(P), dim3(THREADS), 0, s, d_tiles, d_pool_off,
-                       d_pool_lid, d_pool_val, ntiles, d_A, d_B, d_C, d_lambda, R, part);
+    residual_lanes(R, [&](auto L) {
+        hipLaunchKernelGGL(residual_tiles_kernel<decltype(L)::value>, dim3(P), dim3(THREADS), 0, s,
+                           d_tiles, d_pool_off, d_pool_lid, d_pool_val, ntiles, d_A, d_B, d_C,
+                           d_lambda, R, part);
+    });
     CPTC_LAUNCHED();
-    hipLaunchKernelGGL(finalize_add_kernel, dim3(1), dim3(64), 0, s, part, P, d_out2);
+    hipLaunchKernelGGL(finalize_add_kernel, dim3(1), dim3(THREADS), 0, s, part, P, d_out2);
     CPTC_LAUNCHED();
     return CPTC_OK;
 }

@@ -210,6 +210,27 @@ def test_residual3_identical_factors(ca, orc, dev, kind, path, R):
     assert abs(res - ores) <= 1e-12 * ores and abs(x2 - ox2) <= 1e-13 * ox2
 
 
+@pytest.mark.parametrize("kind,path", [("blocks", 1), ("zipf", 2)])
+@pytest.mark.parametrize("R", [1, 2, 4, 5, 8, 9, 17, 32, 35, 65])
+def test_residual3_lane_groups(ca, dev, kind, path, R):
+    """The exact residual at the edges of the lane groups (2 or 4 lanes an
+    element, two ranks a lane): the closed form on the handle's own factors."""
+    t = make(ca, kind, 6)
+    with ca.Als3(t, R=R, threshold=0.03, path=path) as h:
+        h.run(1)
+        F = [h.factor(m, unpermuted=True) for m in range(3)]
+        lam = h.lam()
+        res, x2 = h.residual()
+    xhat = np.einsum("r,er,er,er->e", lam, *(F[m][t.idx[m]] for m in range(3)))
+    mag = np.einsum("r,er,er,er->e", np.abs(lam), *(np.abs(F[m][t.idx[m]]) for m in range(3)))
+    ref = float(np.sum((t.val - xhat) ** 2))
+    # |d(v - x)^2| <= 2 |v - x| (R + 4) eps sum |terms|, and the sums' rounding
+    eps = np.finfo(float).eps
+    bound = 2 * (R + 4) * eps * float(np.sum(np.abs(t.val - xhat) * (mag + np.abs(t.val))))
+    assert abs(res - ref) <= bound + 64 * eps * ref
+    assert abs(x2 - float(np.sum(t.val ** 2))) <= 64 * eps * x2
+
+
 @pytest.mark.parametrize("R", [16, 32, 128])
 def test_fused_path_matches_oracle(ca, orc, dev, R, monkeypatch):
     """ALS_FUSED (als.cu:28, 529-555): one merged launch per mode.  MTTKRP of

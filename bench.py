@@ -289,9 +289,9 @@ def main() -> int:
                        if args.fused else
                        "mttkrp3_blk_kernel (FP64 residual, blocked layout, R in (64,128])"
                        if blocked else
-                       "mttkrp3_seg_wave_kernel (FP64 residual view, R in (64,128])"
-                       if 64 < R <= 128 else
-                       ("mttkrp3_seg_lanes_kernel" if R % 2 == 0 and R <= 64
+                       "mttkrp3_seg_wave_kernel (FP64 residual view, R > 64)"
+                       if 64 < R <= 8000 else
+                       ("mttkrp3_seg_lanes_kernel" if 2 <= R <= 64
                         else "mttkrp3_seg_kernel") +
                        (" (FP64 view of every nonzero: residual + dense pool)" if merged_fp64
                         else " (FP64 residual view)")) + ", per launch = one mode",

@@ -5,13 +5,18 @@
 // FtV[blk_row[b], r] += acc_r (one atomic per (row, rank, segment), skipped
 // when acc_r == 0).  Any R >= 1.
 //
-// Mapping.  A lane owns VEC consecutive ranks (VEC = 2: one 16-byte load per
-// factor row per lane, so a wave reads a 1 KB R=128 row as 64 x 16 B fully
-// coalesced).  LPE = RT / VEC lanes cover one element's rank tile RT; a wave
-// carries EPW = 64 / LPE element slots ("rank-dependent element packing":
-// R=128 -> 1, 64 -> 2, 32 -> 4, 16 -> 8, 8 -> 16 slots per wave).  Partial
-// sums meet in registers (xor-shuffles across the EPW slots of a wave) and
-// then in LDS across waves.  R > RT runs RT-wide rank blocks on grid.y.
+// Mapping.  A lane owns two consecutive ranks (one 16-byte load per factor row
+// per lane, which needs 4-byte alignment only: odd R and 8-byte bases
+// included), so a wave reads a 1 KB R=128 row as 64 x 16 B fully coalesced.
+// LPE = RT / 2 lanes cover one element's rank tile RT; a wave carries EPW = 64 /
+// LPE element slots ("rank-dependent element packing": R=128 -> 1, 64 -> 2,
+// 32 -> 4, 16 -> 8, 8 -> 16 slots per wave).  Partial sums meet in registers
+// (xor-shuffles across the EPW slots of a wave) and then in LDS across waves.
+// R > 128 runs RT-wide rank blocks on grid.y.  R = 1 and R > 8000 run
+// mttkrp3_seg_kernel, a rank a lane.
+//
+// 4 M nonzeros, three modes, odd R a rank a lane -> here: R = 17 436 -> 232 us,
+// 25 434 -> 237, 63 682 -> 399, 65 1285 -> 594, 101 1305 -> 636.
 #include <hip/hip_runtime.h>
 
 #include <type_traits>

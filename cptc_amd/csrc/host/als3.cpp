@@ -353,8 +353,8 @@ int init_streams(Als3& h)
     h.overlap = env_flag("ALS_SERIAL") == 0;
     for (hipStream_t* p : {&h.s, &h.s_pinv, &h.s_dense})
         CPTC_HIP(hipStreamCreateWithFlags(p, hipStreamNonBlocking));
-    for (auto& e : h.ev) CPTC_HIP(timing_event(&e));
-    for (auto& e : h.kev) CPTC_HIP(timing_event(&e));
+    for (auto& e : h.ev) CPTC_HIP(hipEventCreate(&e));
+    for (auto& e : h.kev) CPTC_HIP(hipEventCreate(&e));
     for (hipEvent_t* p : {&h.e_fork, &h.e_pinv, &h.e_dense})
         CPTC_HIP(hipEventCreateWithFlags(p, hipEventDisableTiming));
     return CPTC_OK;
@@ -965,7 +965,7 @@ int run(Als3& h, int iters, double* fit_out, float* ms_out, float* mtt_out)
     while (h.ev_pool.size() < PER * size_t(iters))
     {
         hipEvent_t e = nullptr;
-        CPTC_HIP(timing_event(&e));
+        CPTC_HIP(hipEventCreate(&e));
         h.ev_pool.push_back(e);
     }
     if (h.fit_hist_cap < size_t(iters))

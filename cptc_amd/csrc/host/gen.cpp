@@ -625,7 +625,7 @@ struct Gen
         while (ev_pool.size() < need)
         {
             hipEvent_t e = nullptr;
-            CPTC_HIP(cptc::timing_event(&e));
+            CPTC_HIP(hipEventCreate(&e));
             ev_pool.push_back(e);
         }
         CPTC_HIP(hipEventRecord(ev_pool[0], s));
@@ -1071,9 +1071,9 @@ extern "C" int cptc_gen_create(const cptc_coo* coo, const cptc_gen_opts* opts, v
     if (opts->profile)
     {
         g->ev.resize(size_t(2 + 4 * N));
-        for (auto& e : g->ev) GEN_HIP(cptc::timing_event(&e));
+        for (auto& e : g->ev) GEN_HIP(hipEventCreate(&e));
     }
-    for (auto& e : g->kev) GEN_HIP(cptc::timing_event(&e));
+    for (auto& e : g->kev) GEN_HIP(hipEventCreate(&e));
     GEN_HIP(hipStreamSynchronize(s));
 #undef GEN_TRY
 #undef GEN_HIP

@@ -60,13 +60,6 @@ void set_error(const char* fmt, ...);
         if (rc_ != CPTC_OK) return rc_;                                                    \
     } while (0)
 
-// An event that only times: recording it does not write the caches back to
-// system scope (nobody reads memory on its account).
-inline hipError_t timing_event(hipEvent_t* e)
-{
-    return hipEventCreateWithFlags(e, hipEventDisableSystemFence);
-}
-
 inline hipStream_t as_stream(void* s) { return reinterpret_cast<hipStream_t>(s); }
 
 inline unsigned grid_for(size_t n, unsigned block, unsigned cap = 1u << 20)

@@ -618,8 +618,11 @@ int create(const cptc_coo* coo, const cptc_als3_opts* opts, Als3* h)
     // 6. the factors' values, before alloc_buffers reads them for ||X||^2; it
     // waits for the stream, so init's vector outlives the copy
     init.finish();
-    CPTC_HIP(hipMemcpyAsync(h->d_F, init.values.data(), tot * sizeof(double),
-                            hipMemcpyHostToDevice, h->s));
+    // a copy on the null stream, behind h->s: the first one in a process
+    // creates that stream's queue (3 ms), which the first captured iteration
+    // would pay otherwise (256^3, ten iterations 1.6 -> 4.5 ms)
+    CPTC_HIP(hipStreamSynchronize(h->s));
+    CPTC_HIP(hipMemcpy(h->d_F, init.values.data(), tot * sizeof(double), hipMemcpyHostToDevice));
     CPTC_TRY(alloc_buffers(*h));
     choose_graph(*h);
     choose_small_update(*h);

@@ -29,7 +29,7 @@
 //
 // Measured, a solve's launches back to back, before (column Cholesky above R
 // = 64, a workgroup sweep with two barriers a pivot below) and now: R = 16
-// 6.7 -> 4.1 us, 32 11.6 -> 8.9, 64 27.1 -> 22.5, 65 146 -> 20, 100 319 -> 30,
+// 6.8 -> 4.7 us, 32 11.6 -> 9.5, 64 27.1 -> 22.5, 65 146 -> 20, 100 319 -> 30,
 // 128 623 -> 38.5 (768 threads; 512: 41, 1024 spill: 81).
 #pragma once
 
@@ -97,6 +97,14 @@ __device__ __forceinline__ double recip(double p)
     return fma(fma(-p, r, 1.0), r, r);
 }
 
+// 1 / p as the division gives it (one more step: from within an ulp, the
+// rounded quotient), for the same p
+__device__ __forceinline__ double recip_rn(double p)
+{
+    const double r = recip(p);
+    return fma(fma(-p, r, 1.0), r, r);
+}
+
 // Columns K .. 15 of a block's LDL^T (a: becomes D L^T on and above the
 // diagonal, x: L^-1, from the identity).  Column K reaches the lane's rows by
 // row_newbcast (a row of 16 lanes holds one matrix row), rows K of a and x
@@ -145,8 +153,15 @@ __device__ __forceinline__ void sync_wave()
 // after every pivot the matrix is -A^-1.  M x M blocks of 16 x 16 a wave, in
 // the layout above.
 //
-// SweepWave: the whole matrix in one wave, no barriers: column k reaches the
-// lane's rows by row_newbcast, row k its columns by permutes.
+// SweepWave: the whole matrix in one wave, no barriers.  a_kj is taken from
+// column k (a_jk) and the pivot's reciprocal is the rounded one, so every
+// entry goes through the roundings of the plain column sweep and the inverse
+// has its bits (an over-ranked model on the split-bf16 tiles turns a last bit
+// here into 4e-4 of a factor in five iterations).  Column k reaches the lane's
+// rows by row_newbcast; a lane then holds rows 16 i + l / 16 + 4 v of it for
+// every v, keeps v = (l % 16) / 4, and one permute (lane 16 (l % 4) + l % 16)
+// brings it row 16 i + l % 16, its columns' entries.  With row k by permutes
+// and the two-step reciprocal R = 16 took 4.4 us a launch and 32 8.9.
 template <int M>
 struct SweepWave
 {
@@ -157,18 +172,26 @@ struct SweepWave
     {
         constexpr int KB = K / 16, KL = K % 16, VK = KL / 4, QK = KL % 4;
         const double p = readlane_d(a[KB][KB][VK], 16 * QK + KL);
-        double r[M];
+        double c[M][4], r[M];   // a_ik, a_jk
 #pragma unroll
-        for (int j = 0; j < M; ++j) r[j] = bperm_d(a[KB][j][VK], 16 * QK + lr);
+        for (int i = 0; i < M; ++i)
+#pragma unroll
+            for (int v = 0; v < 4; ++v) c[i][v] = row_bcast_d<KL, 0xf>(a[i][KB][v]);
+#pragma unroll
+        for (int j = 0; j < M; ++j)
+        {
+            const double lo = lr < 4 ? c[j][0] : c[j][1], hi = lr < 12 ? c[j][2] : c[j][3];
+            r[j] = bperm_d(lr < 8 ? lo : hi, 16 * (lr % 4) + lr);
+        }
         if (!(p > tau)) ok = 0;
-        const double ip = recip(p);
+        const double ip = recip_rn(p);
         const bool jk = lr == KL, ik = lk == QK;
 #pragma unroll
         for (int i = 0; i < M; ++i)
 #pragma unroll
             for (int v = 0; v < 4; ++v)
             {
-                const double f = row_bcast_d<KL, 0xf>(a[i][KB][v]) * ip;
+                const double f = c[i][v] * ip;
 #pragma unroll
                 for (int j = 0; j < M; ++j)
                 {
@@ -176,7 +199,7 @@ struct SweepWave
                     if (j == KB) x = jk ? f : x;
                     if (i == KB && v == VK)
                     {
-                        double y = r[j] * ip;
+                        double y = a[i][j][v] * ip;
                         if (j == KB) y = jk ? -ip : y;
                         x = ik ? y : x;
                     }

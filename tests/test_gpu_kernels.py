@@ -625,6 +625,44 @@ def test_pinv_block_edges(ca, dev, R):
     assert int(path.numpy()[0]) == 1
 
 
+def column_sweep_inverse(A):
+    """A^-1 by the symmetric sweep, one pivot at a time, every entry formed as
+    a double-precision program forms it from column k: a_ik / a_kk as a_ik
+    times the rounded 1 / a_kk, then one fused multiply-add with a_jk."""
+    from fractions import Fraction as Q
+
+    a = [[float(x) for x in row] for row in A]
+    n = range(len(a))
+    for k in n:
+        ip = 1.0 / a[k][k]
+        col = [a[i][k] for i in n]
+        f = [c * ip for c in col]
+        fq, cq = [Q(x) for x in f], [Q(x) for x in col]
+        a = [[(-ip if j == k else a[i][j] * ip) if i == k else f[i] if j == k else
+              float(Q(a[i][j]) - fq[i] * cq[j]) for j in n] for i in n]
+    return -np.array(a)
+
+
+@pytest.mark.parametrize("R", [1, 2, 8, 15, 16, 17, 25, 32])
+def test_pinv_has_the_column_sweeps_bits(ca, dev, R):
+    """Up to R = 32 the inverse is the column sweep's to the last bit: where
+    the split-bf16 tiles round the factors and the model has fewer components
+    than R, every other rounding here moves the factors by 1e-4."""
+    rng = np.random.default_rng(50 + R)
+    A = np.ones((R, R))
+    for n in (2 * R + 3, 3 * R + 20):
+        f = rng.random((n, R))
+        A *= f.T @ f
+    A = np.tril(A) + np.tril(A, -1).T
+    path = zeros(ca, (1,), np.int32)
+    dA, Ainv = to_dev(ca, A), zeros(ca, (R, R))
+    assert ca.lib.cptc_pinv_sym(dA.data_ptr(), Ainv.data_ptr(), R, path.data_ptr(),
+                                stream(ca)) == 0
+    ca.sync()
+    assert int(path.numpy()[0]) == 0
+    assert np.array_equal(Ainv.numpy(), column_sweep_inverse(A))
+
+
 @pytest.mark.parametrize("R", [24, 64, 100])
 def test_pinv_singular_takes_jacobi_path(ca, orc, dev, R):
     """Rank-deficient FtF: the fast path (register sweep for R <= 64, blocked

@@ -29,7 +29,7 @@
 //
 // Measured, a solve's launches back to back, before (column Cholesky above R
 // = 64, a workgroup sweep with two barriers a pivot below) and now: R = 16
-// 6.8 -> 4.7 us, 32 11.6 -> 9.5, 64 27.1 -> 22.5, 65 146 -> 20, 100 319 -> 30,
+// 6.8 -> 4.7 us, 32 11.6 -> 9.7, 64 27.1 -> 22.5, 65 146 -> 20, 100 319 -> 30,
 // 128 623 -> 38.5 (768 threads; 512: 41, 1024 spill: 81).
 #pragma once
 
@@ -206,6 +206,8 @@ struct SweepWave
                     a[i][j][v] = x;
                 }
             }
+        if constexpr (K % 4 == 3)
+            if (!ok) return;   // declined: the Jacobi path follows
         if constexpr (K + 1 < 16 * M)
             if (K + 1 < R) from<K + 1>(R, lr, lk, tau, ok);
     }

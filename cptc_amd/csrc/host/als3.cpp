@@ -973,9 +973,9 @@ int run(Als3& h, int iters, double* fit_out, float* ms_out, float* mtt_out)
     }
     if (h.fit_hist_cap < size_t(iters))
     {
-        if (h.d_fit_hist) CPTC_HIP(hipFree(h.d_fit_hist));
+        dev_free(h.d_fit_hist);
         h.d_fit_hist = nullptr;
-        CPTC_HIP(hipMalloc(&h.d_fit_hist, size_t(2) * iters * sizeof(double)));
+        CPTC_TRY(dev_alloc(&h.d_fit_hist, size_t(2) * iters * sizeof(double)));
         h.fit_hist_cap = size_t(iters);
     }
     // kernel events (a few microseconds of idle GPU each) on every 8th
@@ -1244,7 +1244,7 @@ extern "C" int cptc_als3_gather_probe(void* handle, int reps, double* out3)
         cptc::set_error("cptc_als3_gather_probe: %s", hipGetErrorString(e));
         rc = CPTC_ERR_HIP;
     };
-    hipError_t e = hipMalloc(&sink, sizeof(double));
+    hipError_t e = cptc::dev_malloc(reinterpret_cast<void**>(&sink), sizeof(double));
     if (e == hipSuccess) e = hipEventCreate(&e0);
     if (e == hipSuccess) e = hipEventCreate(&e1);
     if (e != hipSuccess) fail(e);

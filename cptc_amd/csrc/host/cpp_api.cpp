@@ -21,6 +21,7 @@
 #include "common.hpp"
 #include "compute_fit.hpp"
 #include "cptc_hip.h"
+#include "dev_pool.hpp"
 #include "dense.hpp"
 #include "generic.hpp"
 #include "host_util.hpp"
@@ -50,7 +51,7 @@ template <class T>
 T* dalloc(size_t n)
 {
     T* p = nullptr;
-    if (n) CHECK_HIP(hipMalloc(reinterpret_cast<void**>(&p), n * sizeof(T)));
+    if (n) CHECK_HIP(cptc::dev_malloc(reinterpret_cast<void**>(&p), n * sizeof(T)));
     return p;
 }
 

@@ -1,6 +1,7 @@
 // Device block pool (dev_pool.hpp).
 #include "dev_pool.hpp"
 
+#include <algorithm>
 #include <list>
 #include <mutex>
 #include <unordered_map>
@@ -41,9 +42,11 @@ size_t round_up(size_t b)
     return (b + m - 1) / m * m;
 }
 
-// whether a block of `have` bytes may stand for one of `need` (no more than
-// half as much again is wasted)
-bool fits(size_t have, size_t need) { return have >= need && have - need <= need / 2; }
+// whether a block of `have` bytes may stand for one of `need`
+bool fits(size_t have, size_t need)
+{
+    return have >= need && have - need <= std::min(need / 2, POOL_WASTE_MAX);
+}
 
 // to the idle list; `out`: blocks that it pushes over the limit
 void give(Pool& P, const PoolBlock& b, std::vector<PoolBlock>& out)
@@ -93,13 +96,22 @@ PoolScope::~PoolScope()
     release(out);
 }
 
+hipError_t dev_malloc(void** p, size_t bytes)
+{
+    hipError_t e = hipMalloc(p, bytes);
+    if (e != hipErrorOutOfMemory) return e;
+    (void)hipGetLastError();
+    pool_release();
+    return hipMalloc(p, bytes);
+}
+
 int dev_alloc_bytes(void** p, size_t bytes)
 {
     *p = nullptr;
     PoolScope* sc = tl_scope;
     if (!sc)
     {
-        CPTC_HIP(hipMalloc(p, bytes));
+        CPTC_HIP(dev_malloc(p, bytes));
         return CPTC_OK;
     }
     PoolBlock b;
@@ -118,6 +130,7 @@ int dev_alloc_bytes(void** p, size_t bytes)
         b = sc->freed_[at];
         sc->freed_[at] = sc->freed_.back();
         sc->freed_.pop_back();
+        sc->freed_bytes_ -= b.bytes;
     }
     else
     {
@@ -136,15 +149,15 @@ int dev_alloc_bytes(void** p, size_t bytes)
     if (!b.p)
     {
         lk.unlock();
-        hipError_t e = hipMalloc(&b.p, need);
-        if (e == hipErrorOutOfMemory)
+        b.bytes = need;
+        hipError_t e = dev_malloc(&b.p, need);
+        if (e == hipErrorOutOfMemory && need > bytes && bytes > 0)
         {
             (void)hipGetLastError();
-            pool_trim();
-            e = hipMalloc(&b.p, need);
+            b.bytes = bytes;
+            e = hipMalloc(&b.p, bytes);
         }
         CPTC_HIP(e);
-        b.bytes = need;
         lk.lock();
     }
     P.live[b.p] = b;
@@ -168,8 +181,16 @@ void dev_free(void* p)
     }
     if (!b.p)   // not the pool's
         (void)hipFree(p);
-    else if (tl_scope)
-        tl_scope->freed_.push_back(b);
+    else if (PoolScope* sc = tl_scope)
+    {
+        if (sc->freed_bytes_ + b.bytes > POOL_SCOPE_MAX)
+        {
+            (void)hipFree(p);   // waits by itself
+            return;
+        }
+        sc->freed_.push_back(b);
+        sc->freed_bytes_ += b.bytes;
+    }
     else if (hipDeviceSynchronize() != hipSuccess)   // hipFree's own wait
         (void)hipFree(p);
     else
@@ -194,6 +215,18 @@ void pool_trim()
         P.idle_bytes = 0;
     }
     release(out);
+}
+
+void pool_release()
+{
+    for (PoolScope* sc = tl_scope; sc; sc = sc->prev_)
+    {
+        if (!sc->idle_ && !sc->freed_.empty()) (void)hipStreamSynchronize(sc->s_);
+        release(sc->freed_);
+        sc->freed_.clear();
+        sc->freed_bytes_ = 0;
+    }
+    pool_trim();
 }
 
 }  // namespace cptc

@@ -13,10 +13,17 @@
 // be handed out again in it at once: everything in a scope runs on the
 // scope's one stream, so the next user's work is queued behind the last
 // one's.  When the scope ends, its stream is waited for and the blocks become
-// idle blocks of the process, which any scope may take.  Idle blocks are at
-// most POOL_IDLE_MAX bytes, the oldest go back to the device first, all of a
-// device's go back before an allocation fails, and cptc_dev_trim returns them
-// on request.
+// idle blocks of the process, which any scope may take.
+//
+// What the blocks cost in memory: idle ones are at most POOL_IDLE_MAX bytes
+// (the oldest go back to the device first), a scope's freed ones at most
+// POOL_SCOPE_MAX, and a block handed out is at most half as much again and
+// POOL_WASTE_MAX larger than the rounded size asked for.  Every device allocation of the
+// library goes through dev_malloc or dev_alloc: where the device has no room,
+// the freed blocks of the thread's scopes and all idle ones go back to it and
+// the allocation is tried again (in a scope, then at its unrounded size), so a
+// set-up fails only if it would without the pool, up to that excess of its
+// live blocks.  cptc_dev_trim returns the idle blocks on request.
 #pragma once
 
 #include <hip/hip_runtime_api.h>
@@ -27,6 +34,8 @@
 namespace cptc {
 
 constexpr size_t POOL_IDLE_MAX = size_t(1) << 30;
+constexpr size_t POOL_SCOPE_MAX = size_t(4) << 30;
+constexpr size_t POOL_WASTE_MAX = size_t(8) << 20;
 
 struct PoolBlock
 {
@@ -48,15 +57,20 @@ public:
 private:
     friend int dev_alloc_bytes(void** p, size_t bytes);
     friend void dev_free(void* p);
+    friend void pool_release();
     hipStream_t s_;
     bool idle_;
     PoolScope* prev_;
     std::vector<PoolBlock> freed_;
+    size_t freed_bytes_ = 0;
 };
 
+// hipMalloc, once more after pool_release() where the device has no room
+hipError_t dev_malloc(void** p, size_t bytes);
 int dev_alloc_bytes(void** p, size_t bytes);
 void dev_free(void* p);
-void pool_trim();   // idle blocks of every device back to it
+void pool_trim();      // idle blocks of every device back to it
+void pool_release();   // and the freed ones of this thread's scopes
 
 template <class T>
 int dev_alloc(T** p, size_t bytes)

@@ -1475,7 +1475,7 @@ extern "C" int cptc_gen_selftest(int verbose, int* failures)
     } own;
     own.s = s;
     auto dal = [&](void** d, size_t bytes) -> int {
-        CPTC_HIP(hipMalloc(d, bytes));
+        CPTC_HIP(cptc::dev_malloc(d, bytes));
         own.p.push_back(*d);
         return CPTC_OK;
     };

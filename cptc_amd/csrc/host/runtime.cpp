@@ -8,6 +8,7 @@
 #include <mutex>
 #include <vector>
 
+#include "dev_pool.hpp"
 #include "hip_util.hpp"
 #include "host_util.hpp"
 
@@ -98,7 +99,7 @@ int scratch_get(int slot, size_t bytes, void** out)
         }
         size_t want = bytes < 4096 ? 4096 : bytes;
         want = (want + 4095) & ~size_t(4095);
-        CPTC_HIP(hipMalloc(&b.ptr, want));
+        CPTC_HIP(dev_malloc(&b.ptr, want));
         b.bytes = want;
         ++g_scratch_gen;   // captured graphs that hold the old address are stale
     }
@@ -123,7 +124,7 @@ extern "C" int cptc_dev_malloc(size_t bytes, void** d_ptr)
 {
     CPTC_REQUIRE(d_ptr, CPTC_ERR_ARG, "cptc_dev_malloc: null out pointer");
     *d_ptr = nullptr;
-    CPTC_HIP(hipMalloc(d_ptr, bytes ? bytes : 1));
+    CPTC_HIP(cptc::dev_malloc(d_ptr, bytes ? bytes : 1));
     return CPTC_OK;
 }
 

@@ -9,6 +9,7 @@
 #include <cstdlib>
 
 #include "cptc_hip.h"
+#include "dev_pool.hpp"
 #include "hip_util.hpp"
 
 extern "C" int cptc_sgd3_run(const uint64_t* d_coords, const double* d_vals, uint64_t nnz,
@@ -25,8 +26,8 @@ extern "C" int cptc_sgd3_run(const uint64_t* d_coords, const double* d_vals, uin
     hipStream_t s = cptc::as_stream(stream);
     uint32_t* d_idx = nullptr;
     double* d_loss = nullptr;
-    CPTC_HIP(hipMalloc(&d_idx, size_t(batch) * sizeof(uint32_t)));
-    if (hipMalloc(&d_loss, sizeof(double)) != hipSuccess)
+    CPTC_HIP(cptc::dev_malloc(reinterpret_cast<void**>(&d_idx), size_t(batch) * sizeof(uint32_t)));
+    if (cptc::dev_malloc(reinterpret_cast<void**>(&d_loss), sizeof(double)) != hipSuccess)
     {
         (void)hipFree(d_idx);
         CPTC_REQUIRE(false, CPTC_ERR_HIP, "cptc_sgd3_run: hipMalloc failed");

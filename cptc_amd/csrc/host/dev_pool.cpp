@@ -71,6 +71,17 @@ void release(const std::vector<PoolBlock>& v)
     for (const PoolBlock& b : v) (void)hipFree(b.p);
 }
 
+// everything queued on device `dev` has finished
+hipError_t device_wait(int dev)
+{
+    int cur = 0;
+    hipError_t e = hipGetDevice(&cur);
+    if (e == hipSuccess && cur != dev) e = hipSetDevice(dev);
+    if (e == hipSuccess) e = hipDeviceSynchronize();
+    if (cur != dev) (void)hipSetDevice(cur);
+    return e;
+}
+
 }  // namespace
 
 PoolScope::PoolScope(hipStream_t s, bool idle) : s_(s), idle_(idle), prev_(tl_scope)
@@ -191,7 +202,7 @@ void dev_free(void* p)
         sc->freed_.push_back(b);
         sc->freed_bytes_ += b.bytes;
     }
-    else if (hipDeviceSynchronize() != hipSuccess)   // hipFree's own wait
+    else if (device_wait(b.dev) != hipSuccess)   // hipFree's own wait
         (void)hipFree(p);
     else
     {

@@ -230,12 +230,40 @@ static void scope_bound()
     CHECK(used[0] <= POOL_IDLE_MAX);
 }
 
+// A block freed outside a scope: its own device is waited for, the caller's
+// current device stays; a scope's blocks wait for its stream
+static void devices()
+{
+    reset(GiB);
+    void* p = nullptr;
+    cur = 1;
+    {
+        PoolScope sc(S);
+        CHECK(dev_alloc_bytes(&p, MiB) == CPTC_OK);
+    }
+    cur = 0;
+    waits[0] = waits[1] = 0;
+    dev_free(p);
+    CHECK(waits[1] == 1 && waits[0] == 0 && cur == 0);
+    CHECK(used[1] == MiB);
+    void* q = nullptr;
+    {
+        PoolScope sc(S);
+        CHECK(dev_alloc_bytes(&q, MiB) == CPTC_OK);   // device 0: not that block
+        CHECK(q != p && used[0] == MiB);
+        dev_free(q);
+        CHECK(stream_waits == 0);
+    }
+    CHECK(stream_waits == 1);
+}
+
 int main()
 {
     setups();
     unrounded();
     others();
     scope_bound();
+    devices();
     reset(GiB);
     std::printf("ok\n");
     std::fflush(stdout);
@@ -260,6 +288,7 @@ def exe(tmp_path_factory):
 
 def test_pool_makes_room(exe):
     """A set-up that fits without the pool fits with it; idle blocks give way
-    to the library's other allocations; what scopes hold back is bounded."""
+    to the library's other allocations; what scopes hold back is bounded; a
+    block's own device is waited for."""
     r = subprocess.run([exe], capture_output=True, text=True, timeout=60)
     assert r.returncode == 0 and r.stdout.strip().endswith("ok"), r.stdout

@@ -509,7 +509,7 @@ __device__ __forceinline__ void chol_factor(const double* __restrict__ FtF, int 
     double x[4], p[4];   // p: A_12, then L21^T
 #pragma unroll
     for (int v = 0; v < 4; ++v)
-        p[v] = (NB == 2 && 16 + lr < R) ? FtF[size_t(lk + 4 * v) * R + 16 + lr] : 0.0;
+        p[v] = (NB == 2 && 16 + lr < R) ? FtF[size_t(16 + lr) * R + lk + 4 * v] : 0.0;
     chol_identity(x, lr, lk);
     chol16_from<0, WIDE, NB == 2>(a[0], x, p, lr, lk, eps, min(R, 16));
     chol_put(w.X[0], x, lr, lk);
@@ -549,7 +549,8 @@ __device__ __forceinline__ void chol_factor(const double* __restrict__ FtF, int 
             }
 }
 
-// Workgroup-wide factorisation, ends with a barrier.
+// Workgroup-wide factorisation of the matrix given by FtF's lower triangle,
+// ends with a barrier.
 template <int NB, bool OUT>
 __device__ __forceinline__ void chol_factor_all(const double* __restrict__ FtF, int R,
                                                 RidgeLds<NB>& w, double* __restrict__ Lout)
@@ -564,7 +565,9 @@ __device__ __forceinline__ void chol_factor_all(const double* __restrict__ FtF, 
             for (int v = 0; v < 4; ++v)
             {
                 const int row = 16 * i + lk + 4 * v, col = 16 * i + lr;
-                a[i][v] = (row < R && col < R) ? FtF[size_t(row) * R + col] : 0.0;
+                a[i][v] = (row < R && col < R)
+                              ? FtF[size_t(max(row, col)) * R + min(row, col)]
+                              : 0.0;
             }
         const double dg = lane < R ? FtF[size_t(lane) * R + lane] : 0.0;
         const double t =

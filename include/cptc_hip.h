@@ -757,7 +757,8 @@ int cptc_gen_unit_scatter(const uint32_t* d_outer_coords, size_t nunits, int nou
 
 /* F = FtV (FtF + eps I)^-1 per row by Cholesky, eps = 1e-12 * tr(FtF) / R +
  * 1e-300 (tr <= 0: 1e-12 + 1e-300); a pivot s <= 0 becomes sqrt(eps).
- * g_chol_solve_kernel, generic.cu:746-819.  R <= 32.  One launch: each
+ * g_chol_solve_kernel, generic.cu:746-819; FtF's lower triangle is read, as
+ * there.  R <= 32.  One launch: each
  * workgroup of 64 rows factors in one wave and solves its rows, with the
  * same bits as cptc_chol_ridge_factor followed by cptc_chol_ridge_apply; no
  * scratch memory. */

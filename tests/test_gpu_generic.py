@@ -513,6 +513,33 @@ def test_chol_ridge_tile_edges(ca, dev, R, rows, scale):
     assert rel_err(outs[1] * sc, outs[0]) <= 64 * R * np.finfo(float).eps * np.linalg.cond(M)
 
 
+@pytest.mark.parametrize("R", [2, 5, 16, 17, 32])
+def test_chol_ridge_reads_the_lower_triangle(ca, orc, dev, R):
+    """generic.cu:746-819 reads FtF's lower triangle only: what stands above the
+    diagonal changes no bit of the factor or of either solve."""
+    rng = np.random.default_rng(R)
+    A = rng.random((3 * R, R))
+    FtF = A.T @ A
+    FtF = np.tril(FtF) + np.tril(FtF, -1).T
+    low = np.tril(FtF) + np.triu(np.full((R, R), np.nan), 1)
+    Y = rng.standard_normal((70, R))
+    got = []
+    for M in (FtF, low):
+        dA, dY, L = dbuf(ca, M), dbuf(ca, Y), ca.DevBuf.zeros((R, R))
+        out, one = ca.DevBuf.zeros((70, R)), ca.DevBuf.zeros((70, R))
+        assert ca.lib.cptc_chol_ridge_factor(dA.data_ptr(), L.data_ptr(), R, None) == 0
+        assert ca.lib.cptc_chol_ridge_apply(L.data_ptr(), dY.data_ptr(), out.data_ptr(), 70, R,
+                                            None) == 0
+        assert ca.lib.cptc_chol_ridge_solve(dA.data_ptr(), dY.data_ptr(), one.data_ptr(), 70, R,
+                                            None) == 0
+        ca.sync()
+        got.append((L.numpy(), out.numpy(), one.numpy()))
+    ref = orc.chol_solve_nd(np.tril(FtF).ravel(), Y.ravel(), R).reshape(70, R)
+    assert rel_err(got[0][2], ref) <= 1e-11
+    for x, y in zip(*got):
+        assert np.array_equal(x, y)
+
+
 def test_chol_ridge_singular_pivot(ca, orc, dev):
     """A rank-deficient FtF hits the s <= 0 -> sqrt(eps) branch."""
     R = 6

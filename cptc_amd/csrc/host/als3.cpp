@@ -164,19 +164,19 @@ int mttkrp_launch(Als3& h, int mode, bool with_pinv)
     if (merged)
     {
         const DevViews3& v = h.views;
-        if (h.timing_kernels) CPTC_HIP(hipEventRecord(h.kev_cur[2 * mode], h.s));
+        if (h.timing_kernels) CPTC_HIP(record_event(h.kev_cur[2 * mode], h.s));
         CPTC_TRY(cptc_mttkrp_merged3_ex(
             mode, h.part.d_tiles4, h.d_tile_f32, size_t(h.part.ntiles), h.d_order[mode],
             h.d_goff[mode], h.ngroups[mode], v.d_coords[mode], v.d_vals[mode], v.d_blk_row[mode],
             v.d_blk_start[mode], v.d_blk_cnt[mode], v.nseg[mode], A, B, C, h.d_FtV, R,
             int(h.dims[0]), int(h.dims[1]), int(h.dims[2]), h.merged_every, h.merged_flags, h.s));
-        if (h.timing_kernels) CPTC_HIP(hipEventRecord(h.kev_cur[2 * mode + 1], h.s));
+        if (h.timing_kernels) CPTC_HIP(record_event(h.kev_cur[2 * mode + 1], h.s));
     }
     else if (dense)
     {
         hipStream_t ds = dense_side ? h.s_dense : h.s;
         if (dense_side) CPTC_HIP(hipStreamWaitEvent(ds, h.e_fork, 0));
-        if (h.timing_kernels) CPTC_HIP(hipEventRecord(h.kev_cur[6 + 2 * mode], ds));
+        if (h.timing_kernels) CPTC_HIP(record_event(h.kev_cur[6 + 2 * mode], ds));
         if (h.tile_b3 && h.timg[mode].ready())
             CPTC_TRY(cptc_mttkrp_dense_tiles3_cws(
                 mode, h.part.d_tiles4, h.timg[mode].cmask, h.timg[mode].segoff,
@@ -194,7 +194,7 @@ int mttkrp_launch(Als3& h, int mode, bool with_pinv)
                 mode, h.part.d_tiles4, h.d_tile_f32, size_t(h.part.ntiles), h.d_order[mode],
                 h.d_goff[mode], h.ngroups[mode], A, B, C, h.d_FtV, R, int(h.dims[0]),
                 int(h.dims[1]), int(h.dims[2]), ds));
-        if (h.timing_kernels) CPTC_HIP(hipEventRecord(h.kev_cur[6 + 2 * mode + 1], ds));
+        if (h.timing_kernels) CPTC_HIP(record_event(h.kev_cur[6 + 2 * mode + 1], ds));
         h.tile_timed[mode] = h.timing_kernels;
         if (dense_side) CPTC_HIP(hipEventRecord(h.e_dense, ds));
     }
@@ -209,7 +209,7 @@ int mttkrp_launch(Als3& h, int mode, bool with_pinv)
         {
             if (!v || !v->ready) continue;
             const bool timed = h.timing_kernels && v == first;
-            if (timed) CPTC_HIP(hipEventRecord(h.kev_cur[2 * mode], h.s));
+            if (timed) CPTC_HIP(record_event(h.kev_cur[2 * mode], h.s));
             if (v == first && h.blk.ready)
             {
                 const DevBlk3& b = h.blk;
@@ -224,7 +224,7 @@ int mttkrp_launch(Als3& h, int mode, bool with_pinv)
                                              v->d_blk_row[mode], v->d_blk_start[mode],
                                              v->d_blk_cnt[mode], v->nseg[mode], F1, F2, h.d_FtV,
                                              R, h.s));
-            if (timed) CPTC_HIP(hipEventRecord(h.kev_cur[2 * mode + 1], h.s));
+            if (timed) CPTC_HIP(record_event(h.kev_cur[2 * mode + 1], h.s));
         }
     }
     if (h.overlap && with_pinv) CPTC_HIP(hipStreamWaitEvent(h.s, h.e_pinv, 0));
@@ -405,7 +405,8 @@ void destroy(Als3* h)
         if (e) (void)hipEventDestroy(e);
     for (hipEvent_t e : {h->e_fork, h->e_pinv, h->e_dense})
         if (e) (void)hipEventDestroy(e);
-    for (hipEvent_t e : h->ev_pool) (void)hipEventDestroy(e);
+    for (hipEvent_t e : h->ev_pool)
+        if (e) (void)hipEventDestroy(e);
     if (h->gexec) (void)hipGraphExecDestroy(h->gexec);
     for (hipStream_t st : {h->s, h->s_pinv, h->s_dense})
         if (st) (void)hipStreamDestroy(st);
@@ -752,7 +753,7 @@ int enqueue_iteration(Als3& h, double* d_out, bool events = true)
 {
     const int R = h.R;
     const size_t RR = size_t(R) * R;
-    if (events) CPTC_HIP(hipEventRecord(h.ev_cur[0], h.s));
+    if (events) CPTC_HIP(record_event(h.ev_cur[0], h.s));
     bool fit_done = false;
     for (int mode = 0; mode < 3; ++mode)
     {
@@ -769,17 +770,17 @@ int enqueue_iteration(Als3& h, double* d_out, bool events = true)
             h.ainv_for = -1;
         }
         h.ftf_for = -1;
-        if (events) CPTC_HIP(hipEventRecord(h.ev_cur[1 + 2 * mode], h.s));
+        if (events) CPTC_HIP(record_event(h.ev_cur[1 + 2 * mode], h.s));
         CPTC_TRY(mttkrp_launch(h, mode, true));
-        if (events) CPTC_HIP(hipEventRecord(h.ev_cur[2 + 2 * mode], h.s));
+        if (events) CPTC_HIP(record_event(h.ev_cur[2 + 2 * mode], h.s));
         CPTC_TRY(update_mode(h, mode, d_out, &fit_done));
     }
     // Gram fit (als.cu:659-715); FtV holds mode C's MTTKRP.  ev_cur[8]:
     // mode C's update done (als.cu's t_solve), for the ALS_PROFILE line
-    if (events) CPTC_HIP(hipEventRecord(h.ev_cur[8], h.s));
+    if (events) CPTC_HIP(record_event(h.ev_cur[8], h.s));
     if (!fit_done)
         CPTC_TRY(cptc_fit_gram(h.F[2], h.d_FtV, h.dims[2], h.d_lambda, h.d_G, 3, R, d_out, h.s));
-    if (events) CPTC_HIP(hipEventRecord(h.ev_cur[7], h.s));
+    if (events) CPTC_HIP(record_event(h.ev_cur[7], h.s));
     return CPTC_OK;
 }
 
@@ -965,12 +966,7 @@ int run(Als3& h, int iters, double* fit_out, float* ms_out, float* mtt_out)
         return CPTC_OK;
     }
     constexpr size_t PER = 21;   // ev (9) + kev (12) per iteration
-    while (h.ev_pool.size() < PER * size_t(iters))
-    {
-        hipEvent_t e = nullptr;
-        CPTC_HIP(hipEventCreate(&e));
-        h.ev_pool.push_back(e);
-    }
+    if (h.ev_pool.size() < PER * size_t(iters)) h.ev_pool.resize(PER * size_t(iters), nullptr);
     if (h.fit_hist_cap < size_t(iters))
     {
         dev_free(h.d_fit_hist);
@@ -1004,9 +1000,9 @@ int run(Als3& h, int iters, double* fit_out, float* ms_out, float* mtt_out)
                 }
             if (h.graph_mode)
             {
-                CPTC_HIP(hipEventRecord(h.ev_cur[0], h.s));
+                CPTC_HIP(record_event(h.ev_cur[0], h.s));
                 CPTC_HIP(hipGraphLaunch(h.gexec, h.s));
-                CPTC_HIP(hipEventRecord(h.ev_cur[7], h.s));
+                CPTC_HIP(record_event(h.ev_cur[7], h.s));
                 CPTC_HIP(hipMemcpyAsync(h.d_fit_hist + 2 * it, h.d_scal + 2, 2 * sizeof(double),
                                         hipMemcpyDeviceToDevice, h.s));
                 replayed[size_t(it)] = 1;

@@ -409,7 +409,8 @@ struct Gen
         for (auto& e : ev) (void)hipEventDestroy(e);
         for (auto& e : kev)
             if (e) (void)hipEventDestroy(e);
-        for (auto& e : ev_pool) (void)hipEventDestroy(e);
+        for (auto& e : ev_pool)
+            if (e) (void)hipEventDestroy(e);
         dfree(d_fit_hist);
         dfree(d_L);
         dfree(d_usum);
@@ -436,7 +437,7 @@ struct Gen
         if (!zeroed) CPTC_HIP(hipMemsetAsync(d_FtV, 0, dims[n] * size_t(R) * sizeof(double), s));
         const bool in = dense && (inner_mask & (1u << n));
         hipEvent_t* ke = kev_cur + 4 * n;
-        if (timing) CPTC_HIP(hipEventRecord(ke[0], s));
+        if (timing) CPTC_HIP(cptc::record_event(ke[0], s));
         if (in)
         {
             if (w_dirty)
@@ -470,8 +471,8 @@ struct Gen
         const bool usum_path = unit_sums && !in;
         if (timing && !usum_path)
         {
-            CPTC_HIP(hipEventRecord(ke[1], s));
-            CPTC_HIP(hipEventRecord(ke[2], s));
+            CPTC_HIP(cptc::record_event(ke[1], s));
+            CPTC_HIP(cptc::record_event(ke[2], s));
         }
         if (usum_path)
         {
@@ -495,8 +496,8 @@ struct Gen
             }
             if (timing)
             {
-                CPTC_HIP(hipEventRecord(ke[1], s));
-                CPTC_HIP(hipEventRecord(ke[2], s));
+                CPTC_HIP(cptc::record_event(ke[1], s));
+                CPTC_HIP(cptc::record_event(ke[2], s));
             }
             int pos = 0;
             while (units.outer[size_t(pos)] != n) ++pos;
@@ -504,7 +505,7 @@ struct Gen
                                            int(units.outer.size()), pos,
                                            const_cast<const double* const*>(d_Fo), d_usum, R, dims[n],
                                            d_FtV, s));
-            if (timing) CPTC_HIP(hipEventRecord(ke[3], s));
+            if (timing) CPTC_HIP(cptc::record_event(ke[3], s));
             return CPTC_OK;
         }
         const cptc::DevViewN& v = views[n];
@@ -517,7 +518,7 @@ struct Gen
             CPTC_TRY(cptc_mttkrp_seg_nd(N, n, v.d_sc, v.level_modes.data(), v.d_vals, nullptr,
                                         v.nnz, v.d_row, v.d_start, v.d_cnt, v.d_single, v.nseg,
                                         F(), d_FtV, R, s));
-        if (timing) CPTC_HIP(hipEventRecord(ke[3], s));
+        if (timing) CPTC_HIP(cptc::record_event(ke[3], s));
         return CPTC_OK;
     }
 
@@ -622,13 +623,8 @@ struct Gen
         }
         const size_t per = size_t(1 + 4 * N);   // iteration end + kernel events
         const size_t need = 1 + per * size_t(iters);
-        while (ev_pool.size() < need)
-        {
-            hipEvent_t e = nullptr;
-            CPTC_HIP(hipEventCreate(&e));
-            ev_pool.push_back(e);
-        }
-        CPTC_HIP(hipEventRecord(ev_pool[0], s));
+        if (ev_pool.size() < need) ev_pool.resize(need, nullptr);
+        CPTC_HIP(cptc::record_event(ev_pool[0], s));
         const bool want = timing;
         for (int it = 0; it < iters; ++it)
         {
@@ -640,7 +636,7 @@ struct Gen
             timing = want;
             kev_cur = kev;
             CPTC_TRY(rc);
-            CPTC_HIP(hipEventRecord(blk[0], s));
+            CPTC_HIP(cptc::record_event(blk[0], s));
         }
         std::vector<double> h(size_t(2) * iters);
         CPTC_HIP(hipMemcpyAsync(h.data(), d_fit_hist, h.size() * sizeof(double),

@@ -62,6 +62,16 @@ void set_error(const char* fmt, ...);
 
 inline hipStream_t as_stream(void* s) { return reinterpret_cast<hipStream_t>(s); }
 
+// hipEventRecord of an event that its first record creates (a null handle
+// until then): hipEventCreate takes 0.3-1.5 us, and a run records only a
+// part of the events it may need (a replayed iteration 2 of 21).
+inline hipError_t record_event(hipEvent_t& e, hipStream_t s)
+{
+    if (!e)
+        if (const hipError_t rc = hipEventCreate(&e); rc != hipSuccess) return rc;
+    return hipEventRecord(e, s);
+}
+
 inline unsigned grid_for(size_t n, unsigned block, unsigned cap = 1u << 20)
 {
     size_t g = (n + block - 1) / block;

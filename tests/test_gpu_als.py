@@ -684,6 +684,39 @@ def test_cli_profile_line(ca, dev, tmp_path):
         assert lines[lines.index(l) - 1].startswith(f"[ALS] iter {k + 1}/3 ")
 
 
+@pytest.mark.parametrize("graph", ["0", "1"])
+def test_run_lengths_change_on_one_handle(ca, dev, graph, monkeypatch):
+    """Runs of 1, 11, 3 and 18 iterations on one handle: an iteration's place
+    in a run (timed, replayed or neither) changes from run to run, and the
+    events it records with it.  Every time is there and positive, as many
+    iterations have kernel times as were timed (one in eight and a run's last),
+    and the fits are those of a fresh handle's single run to 1e-6."""
+    monkeypatch.setenv("ALS_GRAPH", graph)
+    t = make(ca, "clustered", 9)
+    t4 = ca.synth_zipf((40, 24, 70, 90), (0.0, 0.0, 1.2, 1.2), 60000, 2, 6)
+    runs = (1, 11, 3, 18)
+    timed = sum(sum(it % 8 == 0 or it == n - 1 for it in range(n)) for n in runs)
+    with ca.Als3(t, R=9, threshold=0.03) as h, ca.Als3(t, R=9, threshold=0.03) as one:
+        got = [h.run(n) for n in runs]
+        ref = one.run(sum(runs))[0]
+        assert np.max(np.abs(np.concatenate([g[0] for g in got]) - ref)) <= 1e-6
+        for n, (_, ms, mt) in zip(runs, got):
+            assert np.all(ms > 0)
+            last = [it for it in range(n) if it % 8 == 0 or it == n - 1]
+            assert np.all(mt[last] > 0)
+        sp, al, its = h.kernel_times()
+        assert its == timed and np.all(sp >= 0) and np.all(al > 0)
+    if graph == "1":
+        return
+    with ca.Gen(t4, R=8) as h, ca.Gen(t4, R=8) as one:
+        got = [h.run(n) for n in runs]
+        ref = one.run(sum(runs))[0]
+        assert np.max(np.abs(np.concatenate([g[0] for g in got]) - ref)) <= 1e-6
+        assert all(np.all(g[3] > 0) for g in got)
+        assert h.kernel_times()[2] == sum(sum(it % 8 == 7 or it == n - 1 for it in range(n))
+                                          for n in runs)
+
+
 def test_setup_blocks_reused(ca, dev):
     """The set-up's device blocks pass from one handle to the next: layouts,
     factors and MTTKRPs of tensors of several sizes are the same with fresh

@@ -99,7 +99,8 @@ __global__ __launch_bounds__(256) void gram_partial_kernel(const double* __restr
 // in batches of 8 (40 loads, up to 32 MFMAs), two register sets in turn,
 // with scheduling barriers so a batch's loads issue before the previous
 // batch's MFMAs.  Loads are unconditional: rows past the range read its
-// last row and their A is zeroed when the batch is used; columns past R
+// last row and are zeroed when the batch is used, A and B (an infinity in that
+// row would give NaN against a zero A alone); columns past R
 // read column R - 1 and are not stored.
 typedef double gram_d4 __attribute__((ext_vector_type(4)));
 constexpr int GRAM_B = 8;   // K steps (of 4 rows) per batch
@@ -156,18 +157,29 @@ __global__ __launch_bounds__(256) void gram_mfma_partial_kernel(const double* __
             for (int t = 0; t < 4; ++t) x.b[t][u] = row[colB[t]];
         }
     };
+    constexpr size_t STEP = 4 * GRAM_B;   // rows per batch
     auto compute = [&](size_t i0, const Batch& x) {
+        if (i0 + STEP <= r_hi)   // uniform
+        {
+#pragma unroll
+            for (int u = 0; u < GRAM_B; ++u)
+#pragma unroll
+                for (int t = 0; t < 4; ++t)
+                    acc[t] =
+                        __builtin_amdgcn_mfma_f64_16x16x4f64(x.a[u], x.b[t][u], acc[t], 0, 0, 0);
+            return;
+        }
 #pragma unroll
         for (int u = 0; u < GRAM_B; ++u)
         {
-            const size_t i = i0 + size_t(4 * u + lk);
-            const double a = (i < r_hi) ? x.a[u] : 0.0;
+            const bool in = i0 + size_t(4 * u + lk) < r_hi;
+            const double a = in ? x.a[u] : 0.0;
 #pragma unroll
             for (int t = 0; t < 4; ++t)
-                acc[t] = __builtin_amdgcn_mfma_f64_16x16x4f64(a, x.b[t][u], acc[t], 0, 0, 0);
+                acc[t] = __builtin_amdgcn_mfma_f64_16x16x4f64(a, in ? x.b[t][u] : 0.0, acc[t], 0,
+                                                              0, 0);
         }
     };
-    constexpr size_t STEP = 4 * GRAM_B;   // rows per batch
     Batch P, Q;
     load(r_lo, P);
     for (size_t i0 = r_lo; i0 < r_hi; i0 += 2 * STEP)
@@ -176,7 +188,7 @@ __global__ __launch_bounds__(256) void gram_mfma_partial_kernel(const double* __
         const bool more = i0 + STEP < r_hi;
         if (more) load(i0 + STEP, Q);
         __builtin_amdgcn_sched_barrier(0);
-        compute(i0, P);   // zero A past the range
+        compute(i0, P);   // zeros past the range
         __builtin_amdgcn_sched_barrier(0);
         if (!more) break;
         if (i0 + 2 * STEP < r_hi) load(i0 + 2 * STEP, P);

@@ -550,6 +550,24 @@ def test_gram_one_tile_edges(ca, dev, rows, R):
     assert np.all(np.abs(g - A.T @ A) <= bound)
 
 
+@pytest.mark.parametrize("R", [20, 32, 33, 64, 65, 100])
+@pytest.mark.parametrize("rows", [1, 33, 70, 200])
+def test_gram_infinite_last_row(ca, dev, rows, R):
+    """An infinity in the factor's last row (the row that lanes past the end
+    read) makes its column and row infinite, with the other entries' signs,
+    and nothing NaN."""
+    F = np.random.default_rng(rows + R).standard_normal((rows, R))
+    j = R // 2
+    F[-1, j] = np.inf
+    dF, G = to_dev(ca, F), zeros(ca, (R, R))
+    assert ca.lib.cptc_gram(dF.data_ptr(), rows, R, G.data_ptr(), stream(ca)) == 0
+    ca.sync()
+    g = G.numpy()
+    assert np.array_equal(g[j], np.inf * np.sign(F[-1])) and np.array_equal(g[:, j], g[j])
+    k = np.arange(R) != j
+    assert np.allclose(g[k][:, k], F[:, k].T @ F[:, k], rtol=1e-12, atol=1e-11)
+
+
 @pytest.mark.parametrize("R,dim", [(64, 100), (65, 1), (65, 77), (100, 1000), (127, 63),
                                    (128, 28818), (128, 17), (129, 300)])
 def test_apply_pinv_vs_numpy(ca, dev, R, dim):

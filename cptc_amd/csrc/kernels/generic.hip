@@ -389,9 +389,23 @@ __device__ __forceinline__ double chol_ror_add(double x)
     return x + __builtin_bit_cast(double, (uint64_t(hi) << 32) | lo);
 }
 
-// d = sqrt(p) and quotients v / d, correctly rounded, at half the latency of
-// the general ones: one reciprocal root, each result corrected by its exact
-// residual.  For p in about [2^-900, 2^1000]; WIDE takes the general ones.
+// A pivot's quotients v / d from r = 1 / d rounded, corrected once by the
+// exact residual: within an ulp, at half the latency of the division.  They
+// depend on v and d alone, so a factor read back gives the same X_i as the
+// elimination that made it.
+__device__ __forceinline__ double chol_quot(double v, double d, double r)
+{
+    const double q = v * r;
+    return fma(r, fma(-q, d, v), q);
+}
+
+// d for which they are used; other d take the division
+__device__ __forceinline__ bool chol_mid(double d) { return d >= 0x1p-450 && d <= 0x1p500; }
+
+// d = sqrt(p) by one reciprocal root and its exact residual, and r from that
+// root by two more steps: the first leaves it within an ulp of 1 / d, the
+// second rounds it (for a d of 52 one-bits either neighbour, as in recip_rn).
+// For p in about [2^-900, 2^1000]; WIDE takes the general root.
 template <bool WIDE>
 struct Root
 {
@@ -401,6 +415,7 @@ struct Root
         if constexpr (WIDE)
         {
             d = sqrt(p);
+            r = cptc::bsweep::recip_rn(d);
         }
         else
         {
@@ -410,13 +425,14 @@ struct Root
             d = p * r;
             d = fma(0.5 * r, fma(-d, d, p), d);
             r = fma(r, fma(-d, r, 1.0), r);
+            r = fma(r, fma(-d, r, 1.0), r);
         }
     }
     __device__ __forceinline__ double over(double v) const
     {
-        if constexpr (WIDE) return v / d;
-        const double q = v * r;
-        return fma(r, fma(-q, d, v), q);
+        if constexpr (WIDE)
+            if (!chol_mid(d)) return v / d;
+        return chol_quot(v, d, r);
     }
 };
 
@@ -466,7 +482,8 @@ __device__ __forceinline__ void inv16_from(const double (&a)[4], double (&x)[4],
 {
     using namespace cptc::bsweep;
     constexpr int VK = K / 4, QK = K % 4;
-    const double xs = bperm_d(x[VK], 16 * QK + lr) / readlane_d(a[VK], 16 * QK + K);
+    const double xk = bperm_d(x[VK], 16 * QK + lr), d = readlane_d(a[VK], 16 * QK + K);
+    const double xs = chol_mid(d) ? chol_quot(xk, d, recip_rn(d)) : xk / d;
 #pragma unroll
     for (int v = VK; v < 4; ++v)
     {
@@ -709,7 +726,7 @@ __global__ __launch_bounds__(CHOL_T) void chol_apply_kernel(const double* __rest
 }
 
 // Both in one launch, every workgroup factoring for itself: the same bits
-// (quotients are correctly rounded in both).
+// (chol_quot).
 template <int NB>
 __global__ __launch_bounds__(CHOL_T) void chol_solve_kernel(const double* __restrict__ FtF,
                                                             const double* __restrict__ FtV,

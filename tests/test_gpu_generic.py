@@ -540,6 +540,37 @@ def test_chol_ridge_reads_the_lower_triangle(ca, orc, dev, R):
         assert np.array_equal(x, y)
 
 
+@pytest.mark.parametrize("R", [1, 15, 16, 17, 32])
+@pytest.mark.parametrize("last", [1.0, 1e-3, 1e-6])
+def test_chol_ridge_bits_across_the_cut(ca, dev, R, last):
+    """The fast root (trace from 2^-700, diagonal to 2^900) and the general one
+    give the same bits: FtF scaled by even powers of two on both sides of
+    either cut, the solution unscaled, and factor + apply equal to the solve at
+    every scale.  `last` scales a component that is left of a column repeated
+    in the others, so the last pivot is what cancellation leaves."""
+    rng = np.random.default_rng(300 + R)
+    A = rng.random((3 * R + 5, R))
+    if R > 1:
+        A[:, -1] = A[:, 0] + last * A[:, -1]
+    FtF = A.T @ A
+    Y = rng.standard_normal((70, R))
+    got = []
+    for e in (0, -690, -710, 880, 920):
+        f = 2.0 ** e
+        dA, dY, L = dbuf(ca, FtF * f), dbuf(ca, Y), ca.DevBuf.zeros((R, R))
+        out, one = ca.DevBuf.zeros((70, R)), ca.DevBuf.zeros((70, R))
+        assert ca.lib.cptc_chol_ridge_factor(dA.data_ptr(), L.data_ptr(), R, None) == 0
+        assert ca.lib.cptc_chol_ridge_apply(L.data_ptr(), dY.data_ptr(), out.data_ptr(), 70, R,
+                                            None) == 0
+        assert ca.lib.cptc_chol_ridge_solve(dA.data_ptr(), dY.data_ptr(), one.data_ptr(), 70, R,
+                                            None) == 0
+        ca.sync()
+        assert np.array_equal(out.numpy(), one.numpy()), e
+        got.append((L.numpy() * 2.0 ** (-e // 2), one.numpy() * f))
+    for L, x in got[1:]:
+        assert np.array_equal(L, got[0][0]) and np.array_equal(x, got[0][1])
+
+
 def test_chol_ridge_singular_pivot(ca, orc, dev):
     """A rank-deficient FtF hits the s <= 0 -> sqrt(eps) branch."""
     R = 6

@@ -1164,11 +1164,7 @@ extern "C" int cptc_als3_info_get(void* handle, cptc_als3_info* info)
     info->graph_captures = h->n_captures;
     info->fp64_merged = h->aviews.ready ? 1 : 0;
     for (int m = 0; m < 3; ++m) info->merged_segments[m] = h->aviews.ready ? h->aviews.nseg[m] : 0;
-    // the modes within cptc_update_small3's own limit
     info->small_update = h->small_upd;
-    for (int m = 0; m < 3; ++m)
-        if (h->dims[m] > cptc::UPDATE3_SMALL_MAX_ROWS)
-            info->small_update &= m == 2 ? 3 : ~(1 << m);
     info->tiles_beside = (h->dense_beside && h->use_mfma && h->part.ntiles > 0 && !h->fused) ? 1 : 0;
     return CPTC_OK;
 }

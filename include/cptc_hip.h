@@ -508,9 +508,9 @@ typedef struct cptc_als3_info {
                                  one row-sorted view: one FP64 launch per mode, and the
                                  per-mode sparse kernel time covers every nonzero */
     uint64_t merged_segments[3];  /* segments of that view per mode (0: none) */
-    int small_update;         /* bit m: mode m's update runs as cptc_update_small3 (R <= 32, at
-                                 most 4096 rows; larger factors take the same launches);
-                                 bit 3: mode C's also forms the Gram fit scalars */
+    int small_update;         /* bit m: mode m's update runs as cptc_update_small3's launches
+                                 (R <= 32, any number of rows); bit 3: mode C's also forms
+                                 the Gram fit scalars */
 } cptc_als3_info;
 int cptc_als3_info_get(void* handle, cptc_als3_info* info);
 

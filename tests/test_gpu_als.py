@@ -387,21 +387,26 @@ def test_graph_replay_matches_eager(ca, dev, kind, R, path, fused, monkeypatch):
             h.close()
 
 
+WIDE = {"zipf_wide": (700, 400, 5000), "zipf_wider": (9001, 8193, 20011)}
+
+
 @pytest.mark.parametrize("kind,R,bits", [("clustered", 32, 15), ("clustered", 5, 15),
-                                         ("zipf", 16, 15), ("zipf_wide", 16, 3),
+                                         ("zipf", 16, 15), ("zipf_wide", 16, 15),
+                                         ("zipf_wider", 32, 15), ("zipf_wider", 11, 15),
                                          ("zipf", 33, 0)])
 def test_small_update_matches_separate_launches(ca, dev, kind, R, bits, monkeypatch):
-    """The one-launch update (cptc_update_small3: every mode of at most 4096
-    rows at R <= 32, bit 3 = mode C's launch also forms the fit) against
-    ALS_SMALL_UPDATE=0, which runs the separate apply, Gram, scaling and fit
-    launches, from the same factors: 3 iterations, eager and replayed from
-    the captured graph, within test_graph_replay_matches_eager's bounds
-    (fits 1e-8, factors 1e-6: the MTTKRP's atomic order and the new sums'
-    order differ at 1e-16 and ALS amplifies that; a missing clear of FtV or
-    a stale FtF shows at 1e-3 and more).  zipf_wide's mode C has 5000 rows,
-    so modes A and B take the one launch and mode C the separate ones."""
-    if kind == "zipf_wide":
-        t = ca.synth_zipf((700, 400, 5000), (1.1, 1.1, 1.1), 120000, 0, 5)
+    """cptc_update_small3's launches (every mode at R <= 32; bit 3 = mode C's
+    also form the fit) against ALS_SMALL_UPDATE=0, which runs the separate
+    apply, Gram, scaling and fit launches, from the same factors: 3
+    iterations, eager and replayed from the captured graph, within
+    test_graph_replay_matches_eager's bounds (fits 1e-8, factors 1e-6: the
+    MTTKRP's atomic order and the new sums' order differ at 1e-16 and ALS
+    amplifies that; a missing clear of FtV or a stale FtF shows at 1e-3 and
+    more).  zipf_wide's mode C has 5000 rows (32 workgroups, one or two row
+    blocks a wave), zipf_wider's modes have 8193 to 20011 (up to 64
+    workgroups, two or three row blocks a wave)."""
+    if kind in WIDE:
+        t = ca.synth_zipf(WIDE[kind], (1.1, 1.1, 1.1), 120000, 0, 5)
     else:
         t = make(ca, kind, 5)
     hs = {}
@@ -429,6 +434,30 @@ def test_small_update_matches_separate_launches(ca, dev, kind, R, bits, monkeypa
     finally:
         for h in hs.values():
             h.close()
+
+
+@pytest.mark.parametrize("dims", [(4097, 8192, 8193), (16384, 20011, 32767)])
+@pytest.mark.parametrize("R", [7, 16, 25, 32])
+def test_small_update_wide_modes(ca, dev, dims, R, monkeypatch):
+    """One iteration from well-conditioned factors, cptc_update_small3's
+    launches against the separate ones, at the row counts where the number of
+    workgroups changes (32 up to 8192 rows, 64 above) and their waves' last
+    row blocks are ragged: factors, lambda and fit within 1e-11 (a dropped or
+    doubled row block shows at 1e-4 and more)."""
+    t = ca.synth_zipf(dims, (0.6, 0.6, 0.6), 60000, 0, 8)
+    rng = np.random.default_rng(R)
+    F = [rng.standard_normal((d, R)) for d in dims]
+    out = []
+    for small in ("0", "1"):
+        monkeypatch.setenv("ALS_SMALL_UPDATE", small)
+        with ca.Als3(t, R=R, path=2) as h:
+            assert int(h.info.small_update) == (0 if small == "0" else 15)
+            for m in range(3):
+                h.set_factor(m, F[m])
+            fit = h.run(1)[0]
+            out.append([h.factor(m) for m in range(3)] + [h.lam(), fit])
+    for a, b in zip(*out):
+        assert rel_err(a, b) <= 1e-11
 
 
 def test_graph_recaptured_after_scratch_growth(ca, dev, monkeypatch):

@@ -869,9 +869,10 @@ def test_gram_normalize_absorb_next(ca, dev, R, rows):
                                     (3, 129), (32, 4096), (7, 3001), (24, 70), (9, 200)])
 def test_update_small3_matches_steps(ca, dev, R, rows):
     """cptc_update_small3 (FP64 matrix cores; up to 256 rows one workgroup
-    keeps the factor in registers, above that one 16-row block per wave and
-    the last workgroup to finish sums the partials and scales) against the
-    separate calls it replaces: cptc_apply_pinv with lambda, then
+    keeps the factor in registers, above that three launches: one 16-row
+    block per wave, one workgroup that sums their partials, and the scaling
+    with the next pseudoinverse beside it) against the separate calls it
+    replaces: cptc_apply_pinv with lambda, then
     cptc_gram_normalize_absorb_next with the next FtF, then cptc_fit_gram on
     the new factor with grams (G_0, G_1, this G), then cptc_pinv_sym of the
     next FtF.  Factor, norms, lambda, G and FtF within 1e-13 (relative,
@@ -885,8 +886,7 @@ def test_update_small3_matches_steps(ca, dev, R, rows):
     (norm < 1e-14): F, lambda and the Gram's row and column are exactly 0.
     FtV[0, nzero) is cleared after its reads and the rest is untouched; a
     call without fit, next FtF or clearing leaves those alone.  Sizes past
-    4096 rows or R = 33 are refused.  Calls in a row check that the
-    workgroup counter is left at zero."""
+    4096 rows or R = 33 are refused.  Calls in a row give the same."""
     rng = np.random.default_rng(R * 1000 + rows)
     Y = rng.standard_normal((rows, R))
     A = rng.standard_normal((R, R))

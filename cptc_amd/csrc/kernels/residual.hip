@@ -16,28 +16,37 @@ constexpr int THREADS = 256;
 
 // A lane group of LPE lanes takes an element, lane q of it the rank pairs q, q
 // + LPE, ...: with a lane an element every load touches 64 lines.  p0 and p1
-// are the even and the odd ranks' sums.  The whole call, before (a lane an
-// element, one thread adding the partials) and now: 1 M nonzeros R = 8 189 ->
-// 84 us, 16 253 -> 116, 32 354 -> 192; R = 64, 2 M nonzeros 765 -> 466.
+// are the even and the odd ranks' sums.  The whole call, a lane an element
+// with one thread adding the partials -> this: 15.1 M nonzeros in dense tiles
+// R = 8 339 -> 176 us, 16 529 -> 296, 25 567 -> 510, 32 841 -> 505, 100 1654 ->
+// 1390; a view of 2 M power-law nonzeros R = 8 131 -> 51, 32 230 -> 98, 64 354
+// -> 158; 3 M flatter ones R = 32 512 -> 160.
 template <int LPE>
 __device__ double model_value(const double* __restrict__ pa, const double* __restrict__ pb,
                               const double* __restrict__ pc, const double* __restrict__ lam, int R,
                               int q)
 {
     double p0 = 0.0, p1 = 0.0;
-    for (int r = 2 * q; r < R; r += 2 * LPE)
+    int r = 2 * q;
+    // whole pairs only: a condition on the second rank keeps the compiler from
+    // joining a row's two loads
+    for (; r + 1 < R; r += 2 * LPE)
     {
-        const bool two = r + 1 < R;
-        const int r1 = two ? r + 1 : r;
         double x0 = pa[r] * pb[r] * pc[r];
-        double x1 = pa[r1] * pb[r1] * pc[r1];
+        double x1 = pa[r + 1] * pb[r + 1] * pc[r + 1];
         if (lam)
         {
             x0 *= lam[r];
-            x1 *= lam[r1];
+            x1 *= lam[r + 1];
         }
         p0 += x0;
-        if (two) p1 += x1;
+        p1 += x1;
+    }
+    if (r < R)   // the last rank of an odd R
+    {
+        double x = pa[r] * pb[r] * pc[r];
+        if (lam) x *= lam[r];
+        p0 += x;
     }
     double p = p0 + p1;
 #pragma unroll
@@ -155,13 +164,16 @@ __global__ void unpermute_kernel(const double* __restrict__ src, double* __restr
     }
 }
 
-// lanes an element.  1 M nonzeros, the whole call at 1 / 2 / 4 / 8 lanes: R = 4
-// 62 / 63 / 84 / 138 us, 8 98 / 84 / 83 / 133, 16 211 / 150 / 116 / 134, 32 391 /
-// 258 / 192 / 210 (more lanes, fewer elements in flight and more shuffles)
+// lanes an element.  The whole call at 1 / 2 / 4 lanes: 15.1 M nonzeros in
+// dense tiles (rows from L1) R = 4 100 / 114 / 189 us, 8 178 / 176 / 193, 12
+// 225 / 230 / 290, 16 373 / 319 / 296, 32 685 / 585 / 505; 3 M flat power-law
+// nonzeros in a view R = 4 71 / 57 / 66, 8 115 / 80 / 68, 12 160 / 104 / 102,
+// 16 211 / 128 / 97, 32 390 / 234 / 160 (more lanes, fewer lines a load, but
+// fewer elements in flight and more shuffles)
 template <class Run>
 void residual_lanes(int R, Run run)
 {
-    if (R <= 4) run(std::integral_constant<int, 2>{});
+    if (R <= 12) run(std::integral_constant<int, 2>{});
     else run(std::integral_constant<int, 4>{});
 }
 

@@ -211,7 +211,7 @@ def test_residual3_identical_factors(ca, orc, dev, kind, path, R):
 
 
 @pytest.mark.parametrize("kind,path", [("blocks", 1), ("zipf", 2)])
-@pytest.mark.parametrize("R", [1, 2, 4, 5, 8, 9, 17, 32, 35, 65])
+@pytest.mark.parametrize("R", [1, 2, 4, 5, 8, 9, 12, 13, 17, 32, 35, 65])
 def test_residual3_lane_groups(ca, dev, kind, path, R):
     """The exact residual at the edges of the lane groups (2 or 4 lanes an
     element, two ranks a lane): the closed form on the handle's own factors."""

@@ -14,7 +14,7 @@
 //     an iteration.  ALS_SERIAL=1 queues everything on the main stream;
 //   * Grams are cached per mode and refreshed right after that mode's update
 //     (the reference recomputes the same matrices from the same factors);
-//   * the solve is an on-device pseudoinverse (Cholesky inverse with an exact
+//   * the solve is an on-device pseudoinverse (SPD sweep with an exact
 //     Jacobi fallback) instead of cuSOLVER gesvdj.
 #include <hip/hip_runtime_api.h>
 
@@ -134,7 +134,7 @@ struct Als3
 
 // FtV = MTTKRP of `mode`; with_pinv also writes pinv(FtF) to d_Ainv (FtF
 // must already hold the mode's Hadamard product) unless the previous mode's
-// one-launch update formed it already.  Everything is ordered on the main
+// update (update3_small) formed it already.  Everything is ordered on the main
 // stream when this returns.
 int mttkrp_launch(Als3& h, int mode, bool with_pinv)
 {
@@ -246,13 +246,6 @@ bool want_fp64_merge(const Als3& h)
     return !h.use_mfma && h.part.ntiles > 0 && h.part.sparse_nnz > 0;
 }
 
-// Side streams only pay when both sides of the fork run long: each fork /
-// join costs ~20 us of cross-queue waits here.  Measured on MI355X: config 1
-// (tiles only, R = 32) 0.31 ms per iteration overlapped vs 0.26 serial,
-// config 2 (3 M FP64 nonzeros, R = 32) equal, config 3 (37.8 M FP64
-// nonzeros + 82 k tiles, R = 128) 11.7 vs 15.5.  Overlap when the FP64
-// MTTKRP streams at least 2^28 nonzero-ranks or the pseudoinverse takes the
-// blocked Cholesky (R > 64, >= 0.1 ms); ALS_SERIAL=1 forces one stream.
 // ALS_FUSED (als.cu:28, 529-555): the merged single-grid launch when both
 // halves exist; the reference also requires R == 32, here any even R <= 128
 // (16-byte factor rows, the grouped tile role's LDS).
@@ -341,6 +334,18 @@ void choose_small_update(Als3& h)
     if ((h.small_upd & 4) && !(h.o.verbose && std::getenv("ALS_DEBUG"))) h.small_upd |= 8;
 }
 
+// Side streams only pay when both sides of the fork run long: each fork /
+// join costs ~20 us of cross-queue waits here.  Measured on MI355X: config 1
+// (tiles only, R = 32) 0.31 ms per iteration overlapped vs 0.26 serial,
+// config 2 (3 M FP64 nonzeros, R = 32) equal, config 3 (37.8 M FP64
+// nonzeros + 82 k tiles, R = 128) 11.7 vs 15.5.  Overlap when the FP64
+// MTTKRP streams at least 2^28 nonzero-ranks, or at R > 64, where the
+// pseudoinverse is two launches (20-39 us and the Jacobi kernel's check of the
+// first one's verdict) that the fork hides behind the MTTKRP: ms per
+// iteration on one stream / forked, R = 65 0.220 / 0.215 at 20 k nonzeros,
+// 0.330 / 0.299 at 0.8 M, 0.417 / 0.417 at 2 M; R = 100 0.301 / 0.246, 0.484 /
+// 0.349, 0.552 / 0.517, 1.109 / 1.081 at 8 M; R = 128 0.332 / 0.279, 0.511 /
+// 0.358, 0.590 / 0.531, 1.195 / 1.136.  ALS_SERIAL=1 forces one stream.
 void choose_overlap(Als3& h)
 {
     const double work = double(h.views.nnz + h.dviews.nnz) * double(h.R);
@@ -680,7 +685,7 @@ int alloc_buffers(Als3& hr)
 }
 
 // d_fit: where the iteration's fit scalars go; *fit_done is set when this
-// update formed them (mode C on the one-launch path).
+// update formed them (mode C by update3_small).
 int update_mode(Als3& h, int mode, double* d_fit = nullptr, bool* fit_done = nullptr)
 {
     const int R = h.R;
@@ -786,8 +791,8 @@ int enqueue_iteration(Als3& h, double* d_out, bool events = true)
 
 // The state an iteration leaves behind and finds: every Gram current, mode
 // 0's FtF formed by mode 2's update and FtV not yet cleared for mode 0 (the
-// fit reads it), or already cleared when mode C's one-launch update formed
-// the fit, and mode 0's pinv formed by that launch too.  Only an iteration
+// fit reads it), or already cleared when mode C's update3_small formed the
+// fit, and mode 0's pinv formed by that update too.  Only an iteration
 // that starts there has the captured iteration's launches.
 bool steady(const Als3& h)
 {

@@ -82,9 +82,9 @@ __global__ __launch_bounds__(256) void gram_partial_kernel(const double* __restr
 
 // Gram partials for R > 32 on the FP64 matrix cores (v_mfma_f64_16x16x4f64);
 // cptc_gram at R = 64 with this instead of the 16 x 16 threads above, and the
-// partials' sum below over four waves: 64 rows 12.9 -> 8.7 us, 1500 14.6 ->
-// 10.6, 12000 25.6 -> 14.5, 32768 39 -> 18 (R = 100, the sum alone: 12000 28.7
-// -> 22.6, 32768 41.6 -> 32.7).  At R <= 32 a tile's MFMAs are mostly padding
+// partials' sum below over four waves: 64 rows 13.3 -> 8.6 us, 1500 14.1 ->
+// 10.8, 12000 25.5 -> 14.5, 32768 36.8 -> 17.7 (R = 100, the sum and whole
+// batches without selects: 12000 28.7 -> 22.4, 32768 41.5 -> 29.9).  At R <= 32 a tile's MFMAs are mostly padding
 // and the threads have 1 or 4 entries: 500 rows 7.8 us at R = 32 there.
 //
 // grid.x = row range p (rows [p rpw, (p + 1) rpw)), grid.y = one upper-
@@ -2070,9 +2070,9 @@ int update3_small(double* d_FtV, double* d_Ainv, double* d_F, size_t rows, int R
     }
     const int nr = int(rows), nz = int(nzero);
     // one workgroup up to 256 rows, three launches above that
-    // (CPTC_UPD3_ONE_ROWS overrides the limit, at most 512; 0 = never).  At R =
-    // 32, 256 rows take 13.0 us in one workgroup and 22 in three launches;
-    // 512 rows 22.0 in either.
+    // (CPTC_UPD3_ONE_ROWS overrides the limit, at most 512; 0 = never).  With
+    // fit and next pseudoinverse, one workgroup / three launches: 256 rows 9.6 /
+    // 14.4 us at R = 16, 19.2 / 20.4 at 25, 21.0 / 22.8 at 32.
     static const int one_rows = [] {
         const char* e = std::getenv("CPTC_UPD3_ONE_ROWS");
         return e ? std::atoi(e) : 256;

@@ -410,7 +410,7 @@ int cptc_sgd3_run(const uint64_t* d_coords, const double* d_vals, uint64_t nnz, 
                   double* batch_rmse, void* stream);
 
 /* Writes pinv(FtF) (R x R) to d_Ainv with the same rule as cptc_solve_pinv;
- * *d_path (device int, may be NULL) receives 0 = Cholesky, 1 = Jacobi. */
+ * *d_path (device int, may be NULL) receives 0 = the SPD fast path, 1 = Jacobi. */
 int cptc_pinv_sym(const double* d_FtF, double* d_Ainv, int R, int* d_path, void* stream);
 
 /* F = FtV * Ainv (row-major dim x R), then F[:, r] /= div[r] when d_div !=

@@ -491,8 +491,10 @@ def test_chol_ridge_factor_apply(ca, dev, R, rows, rank_def):
 def test_chol_ridge_tile_edges(ca, dev, R, rows, scale):
     """The 16-row tiles and 16-column blocks at their edges, more rows than
     one pass takes, in place, and scales on both sides of the range of the
-    fast root and quotient (powers of two, so the result only scales: same
-    bits as at scale 1, where the solve's backward error is <= c R eps)."""
+    fast root and quotient (powers of two, so the result only scales, up to
+    the 1e-300 in eps and to results near the smallest numbers: within the
+    forward bound of the result at scale 1, whose backward error is <= c R
+    eps)."""
     rng = np.random.default_rng(R + rows)
     A = rng.random((3 * R + 5, R))
     FtF = A.T @ A

@@ -607,7 +607,7 @@ def test_solve_pinv_spd(ca, dev, R):
     assert ca.lib.cptc_solve_pinv(dA.data_ptr(), dY.data_ptr(), out.data_ptr(), dim, R,
                                   dl.data_ptr(), stream(ca)) == 0
     ca.sync()
-    assert int(path.numpy()[0]) == 0                    # Cholesky fast path
+    assert int(path.numpy()[0]) == 0                    # the fast path
     inv = np.linalg.inv(A)
     assert rel_err(Ainv.numpy(), inv) < 1e-9
     assert rel_err(out.numpy(), (Y @ inv) / lam) < 1e-9
@@ -683,8 +683,8 @@ def test_pinv_has_the_column_sweeps_bits(ca, dev, R):
 
 @pytest.mark.parametrize("R", [24, 64, 100])
 def test_pinv_singular_takes_jacobi_path(ca, orc, dev, R):
-    """Rank-deficient FtF: the fast path (register sweep for R <= 64, blocked
-    Cholesky above) hands over to the Jacobi pseudoinverse."""
+    """Rank-deficient FtF: the fast path (one-wave sweep for R <= 32, four-wave
+    sweep to 64, block sweep above) hands over to the Jacobi pseudoinverse."""
     rng = np.random.default_rng(3)
     F = rng.random((max(60, 2 * R), R))
     F[:, 7] = F[:, 3]

@@ -317,7 +317,7 @@ void choose_graph(Als3& h)
 }
 
 // R <= 32: a mode's apply, Gram, norms, normalisation, scaling, the next
-// mode's FtF and its pseudoinverse in one launch (up to 256 rows) or three
+// mode's FtF and its pseudoinverse in one launch (up to 256-512 rows) or three
 // instead of six, and mode C's with the Gram fit and the clearing of FtV for
 // mode A (two launches fewer again).  256^3, R = 32: 0.198 ms per iteration
 // with the separate launches, 0.151 with one; 9000 x 5003 x 28000 at R = 25

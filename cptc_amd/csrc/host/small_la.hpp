@@ -30,8 +30,8 @@ int gram_normalize_absorb_next_tail(double* d_F, size_t rows, int R, double* d_G
                                     double* d_FtF, const TailJobs* t, hipStream_t s);
 
 // cptc_update_small3 for any number of rows (R <= 32): a mode's whole update
-// in one launch up to 256 rows, in three above.  The entry point takes at most
-// UPDATE3_SMALL_MAX_ROWS.
+// in one launch up to 256 rows (512 at R <= 16), in three above.  The entry
+// point takes at most UPDATE3_SMALL_MAX_ROWS.
 constexpr size_t UPDATE3_SMALL_MAX_ROWS = 4096;
 int update3_small(double* d_FtV, double* d_Ainv, double* d_F, size_t rows, int R, double* d_G,
                   double* d_norms, double* d_lambda, const double* d_other, double* d_FtF,

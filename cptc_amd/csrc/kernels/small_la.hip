@@ -1372,8 +1372,8 @@ int scale_launch(double* F, size_t rows, int R, const double* norms, const cptc:
 //   scale: the factor scaled in place and FtV cleared over the whole chip,
 //     the pinv in a workgroup of its own beside them.
 // The sums run in the matrix cores' order, not the separate kernels'.  Up to
-// 256 rows one workgroup does it all (update3_one_kernel, below).  The form
-// before, one launch whose last workgroup to finish summed, rescaled the
+// 256 rows, at R <= 16 512, one workgroup does it all (update3_one_kernel,
+// below).  The form before, one launch whose last workgroup to finish summed, rescaled the
 // whole factor and formed the pinv, against these three, back to back: R = 25
 // 512 rows 21.1 / 20.2 us, 1000 27.1 / 21.0, 3001 57.4 / 23.7, 4096 73.8 /
 // 24.4; R = 32 at 4096 rows 82.9 / 26.5.
@@ -2069,14 +2069,19 @@ int update3_small(double* d_FtV, double* d_Ainv, double* d_F, size_t rows, int R
         Vw = static_cast<double*>(pb) + RR;
     }
     const int nr = int(rows), nz = int(nzero);
-    // one workgroup up to 256 rows, three launches above that
-    // (CPTC_UPD3_ONE_ROWS overrides the limit, at most 512; 0 = never).  With
-    // fit and next pseudoinverse, one workgroup / three launches: 256 rows 9.6 /
-    // 14.4 us at R = 16, 19.2 / 20.4 at 25, 21.0 / 22.8 at 32.
-    static const int one_rows = [] {
+    // one workgroup up to 256 rows and, at R <= 16 with little of FtV to clear,
+    // 512; three launches above that (CPTC_UPD3_ONE_ROWS overrides the limit, at
+    // most 512; 0 = never).  With fit and next pseudoinverse, one workgroup /
+    // three launches: 256 rows 9.6 / 14.4 us at R = 16, 19.2 / 20.4 at 25, 21.0 /
+    // 22.8 at 32; 300 rows 8.6 / 12.2 at R = 3, 10.6 / 14.8 at 16, 24.3 / 23.0 at
+    // 32; 512 rows 10.6 / 12.6, 13.0 / 14.7, 29.6 / 23.0.  One workgroup clears
+    // alone: 512 rows at R = 16 with 8192 values 15.5 / 16.5, 32 768 18.3 / 16.5,
+    // 524 288 72 / 17.
+    static const int forced = [] {
         const char* e = std::getenv("CPTC_UPD3_ONE_ROWS");
-        return e ? std::atoi(e) : 256;
+        return e ? std::atoi(e) : -1;
     }();
+    const int one_rows = forced >= 0 ? forced : R <= 16 && nz <= 8192 ? 512 : 256;
     if (nr <= one_rows && nr <= 16 * UPD1_WAVES * 4)
     {
         const bool two = nr <= 16 * UPD1_WAVES * 2;

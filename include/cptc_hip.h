@@ -267,7 +267,8 @@ int cptc_gram_normalize_absorb_next(double* d_F, size_t rows, int R, double* d_G
                                     double* d_FtF, void* stream);
 
 /* One mode's whole update for a small factor (1 <= rows <= 4096, R <= 32;
- * FP64 matrix cores) in one launch up to 256 rows, in three above: F = (d_FtV * d_Ainv) /
+ * FP64 matrix cores) in one launch up to 256 rows (512 at R <= 16 with nzero
+ * <= 8192), in three above: F = (d_FtV * d_Ainv) /
  * lambda (cptc_apply_pinv's product with d_Ainv = pinv(FtF) given), then
  * cptc_gram_normalize_absorb_next on it (G, norms, lambda, F scaled, the
  * next FtF = G .* d_other when d_other / d_FtF are given), then

@@ -866,13 +866,15 @@ def test_gram_normalize_absorb_next(ca, dev, R, rows):
 
 @pytest.mark.parametrize("R,rows", [(1, 1), (5, 17), (16, 256), (17, 15), (20, 513),
                                     (31, 1000), (32, 256), (32, 257), (32, 512), (32, 1024),
-                                    (3, 129), (32, 4096), (7, 3001), (24, 70), (9, 200)])
+                                    (3, 129), (32, 4096), (7, 3001), (24, 70), (9, 200),
+                                    (16, 257), (1, 400), (11, 511), (16, 510), (15, 512),
+                                    (16, 513), (17, 257)])
 def test_update_small3_matches_steps(ca, dev, R, rows):
-    """cptc_update_small3 (FP64 matrix cores; up to 256 rows one workgroup
-    keeps the factor in registers, above that three launches: one 16-row
-    block per wave, one workgroup that sums their partials, and the scaling
-    with the next pseudoinverse beside it) against the separate calls it
-    replaces: cptc_apply_pinv with lambda, then
+    """cptc_update_small3 (FP64 matrix cores; up to 256 rows, or 512 at R <=
+    16 with nzero at most 8192, one workgroup keeps the factor in registers,
+    above that three launches: one 16-row block per wave, one workgroup that
+    sums their partials, and the scaling with the next pseudoinverse beside
+    it) against the separate calls it replaces: cptc_apply_pinv with lambda, then
     cptc_gram_normalize_absorb_next with the next FtF, then cptc_fit_gram on
     the new factor with grams (G_0, G_1, this G), then cptc_pinv_sym of the
     next FtF.  Factor, norms, lambda, G and FtF within 1e-13 (relative,
